@@ -266,6 +266,20 @@ int moe_attention_bf16(const void *q, const void *k_cache, const void *v_cache, 
                        const void *pos0_i32, int64_t max_seq, float scaling, void *out,
                        void *stream);
 
+/* The same with a workspace, so that several
+ * workgroups can share a row's keys when the rows alone do not fill the device: one token
+ * behind more than 512 keys, few tokens behind a long context.  Their probabilities are
+ * rounded before the division by the sum (several tokens) or not at all (one token).
+ * moe_attention_workspace_bytes: what any call of 1 .. T tokens needs.  The workspace is
+ * 16-byte aligned and its first 4096 bytes are zero before the first call (every call leaves
+ * them zero); calls that share it must be ordered (one stream).  Null: moe_attention_bf16. */
+int64_t moe_attention_workspace_bytes(int64_t T, int32_t n_q_heads, int32_t n_kv_heads,
+                                      int32_t head_dim, int64_t max_seq);
+int moe_attention_ws_bf16(const void *q, const void *k_cache, const void *v_cache, int64_t T,
+                          int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
+                          const void *pos0_i32, int64_t max_seq, float scaling, void *out,
+                          void *workspace, int64_t workspace_bytes, void *stream);
+
 /* y[T, N] = bf16(x[T, K] W[N, K]^T) with fp32 accumulation, 1 <= T <= 4: the decode-time
  * q/k/v/o projections and lm_head (nn.Linear without bias on bf16 tensors). */
 int moe_gemv_bf16(const void *weight, const void *x, int64_t T, int32_t N, int32_t K, void *y,

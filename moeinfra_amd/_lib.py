@@ -71,6 +71,9 @@ SIGNATURES = {
                          ctypes.c_int),
     "moe_attention_bf16": ([_vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i64, ctypes.c_float,
                             _vp, _vp], ctypes.c_int),
+    "moe_attention_workspace_bytes": ([_i64, _i32, _i32, _i32, _i64], _i64),
+    "moe_attention_ws_bf16": ([_vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _i64, ctypes.c_float,
+                               _vp, _vp, _i64, _vp], ctypes.c_int),
     "moe_gemv_bf16": ([_vp, _vp, _i64, _i32, _i32, _vp, _vp], ctypes.c_int),
     "moe_layer_norm_workspace_bytes": ([_i32, _i32, _i32, _i32], _i64),
     "moe_layer_forward_nf4_norm": ([ctypes.POINTER(MoeNf4Expert), _i32, _vp, _vp, _vp, _vp, ctypes.c_float, _i32, _i32, _i32,

@@ -42,6 +42,18 @@ __device__ __forceinline__ float bf16hi_to_f32(uint32_t w) {
   return __builtin_bit_cast(float, w & 0xffff0000u);
 }
 
+__device__ __forceinline__ float bf16r(float v) { return bf16_to_f32(f32_to_bf16(v)); }
+
+// Eight bf16 values of a 16-byte load as floats.
+__device__ __forceinline__ void unpack8(const uint4 v, float *f) {
+  const uint32_t a[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    f[2 * e] = bf16lo_to_f32(a[e]);
+    f[2 * e + 1] = bf16hi_to_f32(a[e]);
+  }
+}
+
 // ---------------------------------------------------------------- streamed loads
 // 16 bytes of global memory loaded with the non-temporal hint (global_load_dwordx4 ... nt),
 // for weights that a pass reads exactly once.  A single-pass read of 1 GB streams at

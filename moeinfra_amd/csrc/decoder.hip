@@ -8,13 +8,13 @@
 //   add_rmsnorm   r = x (+ residual), out = bf16(w * bf16(r * rsqrt(mean(r^2) + eps)))
 //   rope_kv       q, k rotated (rotate-half convention, cos/sin rounded to bf16) at
 //                 positions pos0 + t; k and v written to the KV cache
-//   attention     grouped-query causal attention of T query rows against the cache
 //   gemv          y = bf16(W x) for up to 4 tokens (the decode projections and lm_head)
 // and the fused single-token forms of a decode step:
 //   qkv_rope      input norm + q/k/v projection + rotary + KV-cache write
 //   head_logits   final norm + lm_head + per-workgroup argmax candidates, and
 //   argmax_finish the token, the generated-id buffer, its counter and the position
-// (the post-attention norm runs inside the MoE layer's gate/up kernel, decode_layer.hip).
+// (attention is in attention.hip; the post-attention norm runs inside the MoE layer's gate/up
+// kernel, decode_layer.hip).
 #include "norm_row.h"
 
 namespace moe {
@@ -33,15 +33,6 @@ add_rmsnorm_kernel(const uint16_t *__restrict__ x, const uint16_t *__restrict__ 
 
 constexpr int kRopeThreads = 256;
 constexpr int kRopeMaxHalf = 256;  // head_dim <= 512
-
-__device__ __forceinline__ void unpack8(const uint4 v, float *f) {
-  const uint32_t a[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    f[2 * e] = bf16lo_to_f32(a[e]);
-    f[2 * e + 1] = bf16hi_to_f32(a[e]);
-  }
-}
 
 // Token t (blockIdx.x) at position pos0 + t.  The hd/2 rotary angles of the position are
 // evaluated once (cos/sin rounded to bf16, as the bf16 module's cos/sin tensors) into LDS;
@@ -99,156 +90,6 @@ rope_kv_kernel(const uint16_t *__restrict__ qkv, int nq, int nkv, int hd,
     const int head = idx / cpr, c = idx - head * cpr;
     *reinterpret_cast<uint4 *>(vc + ((size_t)head * max_seq + pos) * hd + c * 8) =
         *reinterpret_cast<const uint4 *>(vsrc + (size_t)head * hd + c * 8);
-  }
-}
-
-constexpr int kAttnThreads = 256;
-constexpr int kAttnMaxKeys = 8192;
-constexpr int kAttnMaxHeadDim = 256;
-constexpr int kAttnRowsInFlight = 8;  // cache rows per thread per pass
-
-// Scores of the pass starting at key j0 from its loaded K rows: s_p[j] = bf16(bf16(q.k_j) *
-// scaling) for the keys j < nkeys, and the running maximum.  The eight rows' lane partials
-// are formed first and summed over each row's lpr lanes together (DPP within a 16-lane row).
-__device__ __forceinline__ void attn_scores(const uint4 (&kv)[kAttnRowsInFlight], const float (&qf)[8],
-                                            int j0, int nkeys, int rpp, int rr, int lpr, int sub,
-                                            float scaling, float *s_p, float &mx) {
-  float dot[kAttnRowsInFlight];
-#pragma unroll
-  for (int u = 0; u < kAttnRowsInFlight; ++u) {
-    float kf[8];
-    unpack8(kv[u], kf);
-    float d = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) d = fmaf(qf[e], kf[e], d);
-    dot[u] = d;
-  }
-  lane_groups_reduce<false>(dot, lpr);
-#pragma unroll
-  for (int u = 0; u < kAttnRowsInFlight; ++u) {
-    const int j = j0 + u * rpp + rr;
-    const float sc = bf16r(bf16r(dot[u]) * scaling);
-    const bool ok = j < nkeys;
-    mx = ok ? fmaxf(mx, sc) : mx;
-    if (ok && sub == 0) s_p[j] = sc;
-  }
-}
-
-// acc += p_j v_j over the pass's rows j < nkeys, in row order.
-__device__ __forceinline__ void attn_pv(const uint4 (&vv)[kAttnRowsInFlight], int j0, int nkeys,
-                                        int rpp, int rr, const float *s_p, float (&acc)[8]) {
-#pragma unroll
-  for (int u = 0; u < kAttnRowsInFlight; ++u) {
-    const int j = j0 + u * rpp + rr;
-    if (j < nkeys) {
-      const float p = s_p[j];
-      float vf[8];
-      unpack8(vv[u], vf);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) acc[e] = fmaf(p, vf[e], acc[e]);
-    }
-  }
-}
-
-// One workgroup per (query head, token): scores of keys 0 .. pos0 + t (causal), bf16 scores
-// scaled in bf16, fp32 softmax rounded to bf16, then the bf16 probabilities times V with
-// fp32 accumulation.  A cache row of hd bf16 is read by hd/8 consecutive lanes, 16 bytes
-// each, so the workgroup covers rpp = 256/(hd/8) rows per load instruction and a pass takes
-// 8 such loads per thread (128 rows at hd = 128); a score is the xor-shuffle sum over its
-// row's lanes.  The first pass's K and V rows are loaded together with q and the position,
-// before the key count is known (row indexes clamped to the cache, results of rows past the
-// last key discarded), so a context of up to one pass of keys costs one memory round trip;
-// later passes load rows clamped to the last key.
-__global__ void __launch_bounds__(kAttnThreads)
-attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc,
-                 const uint16_t *__restrict__ vc, int nq, int nkv, int hd,
-                 const int32_t *__restrict__ pos0, int64_t max_seq, float scaling,
-                 uint16_t *__restrict__ out) {
-  __shared__ float s_p[kAttnMaxKeys];
-  __shared__ float s_red[kAttnThreads / kWave];
-  __shared__ __attribute__((aligned(16))) float s_acc[kAttnThreads * 8];
-  MOE_ARGS_FIRST(MOE_LIST("+s"(nq), "+s"(nkv), "+s"(hd), "+s"(max_seq), "+s"(scaling)),
-                 MOE_LIST("s"(q), "s"(kc), "s"(vc), "s"(pos0), "s"(out)));
-  const int h = blockIdx.x, t = blockIdx.y;
-  const int kvh = h / (nq / nkv);
-  const int lpr = hd >> 3;               // lanes per row: a power of two <= 32
-  const int rpp = kAttnThreads / lpr;    // rows per load instruction of the workgroup
-  const int npass = kAttnRowsInFlight * rpp;
-  const int sub = threadIdx.x & (lpr - 1), rr = threadIdx.x / lpr;
-  float qf[8];
-  unpack8(*reinterpret_cast<const uint4 *>(q + ((size_t)t * nq + h) * hd + sub * 8), qf);
-  const uint16_t *kbase = kc + (size_t)kvh * max_seq * hd + sub * 8;
-  const uint16_t *vbase = vc + (size_t)kvh * max_seq * hd + sub * 8;
-  uint4 kv[kAttnRowsInFlight], vv[kAttnRowsInFlight];
-#pragma unroll
-  for (int u = 0; u < kAttnRowsInFlight; ++u) {
-    const int j = min(u * rpp + rr, (int)max_seq - 1);
-    kv[u] = *reinterpret_cast<const uint4 *>(kbase + (size_t)j * hd);
-    vv[u] = *reinterpret_cast<const uint4 *>(vbase + (size_t)j * hd);
-  }
-  // Keys 0 .. pos0 + t, bounded by the cache (a position past it is a caller error).
-  const int nkeys = min(*pos0 + t + 1, (int)max_seq);
-  float mx = -INFINITY;
-  attn_scores(kv, qf, 0, nkeys, rpp, rr, lpr, sub, scaling, s_p, mx);
-  for (int j0 = npass; j0 < nkeys; j0 += npass) {
-#pragma unroll
-    for (int u = 0; u < kAttnRowsInFlight; ++u) {
-      const int j = min(j0 + u * rpp + rr, nkeys - 1);
-      kv[u] = *reinterpret_cast<const uint4 *>(kbase + (size_t)j * hd);
-    }
-    attn_scores(kv, qf, j0, nkeys, rpp, rr, lpr, sub, scaling, s_p, mx);
-  }
-  // block max, then the block sum of the exponentials (each a wave reduction, then the
-  // four waves' values through LDS in wave order)
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
-  {
-    float m[1] = {mx};
-    lane_groups_reduce<true>(m, kWave);
-    if (lane == 0) s_red[wave] = m[0];
-    __syncthreads();
-    mx = s_red[0];
-    for (int w = 1; w < kAttnThreads / kWave; ++w) mx = fmaxf(mx, s_red[w]);
-    __syncthreads();
-  }
-  float sum = 0.0f;
-  for (int j = threadIdx.x; j < nkeys; j += kAttnThreads) {
-    const float e = expf(s_p[j] - mx);
-    s_p[j] = e;
-    sum += e;
-  }
-  {
-    float v[1] = {sum};
-    lane_groups_reduce<false>(v, kWave);
-    if (lane == 0) s_red[wave] = v[0];
-    __syncthreads();
-    sum = 0.0f;
-    for (int w = 0; w < kAttnThreads / kWave; ++w) sum += s_red[w];
-    __syncthreads();
-  }
-  for (int j = threadIdx.x; j < nkeys; j += kAttnThreads) s_p[j] = bf16r(s_p[j] / sum);
-  __syncthreads();
-  // out[d] = sum_j p_j v_j[d]: thread (rr, sub) accumulates dims sub*8 .. sub*8+7 over rows
-  // rr, rr + rpp, ... in order; then the rpp partial rows are summed through LDS.
-  float acc[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-  attn_pv(vv, 0, nkeys, rpp, rr, s_p, acc);
-  for (int j0 = npass; j0 < nkeys; j0 += npass) {
-#pragma unroll
-    for (int u = 0; u < kAttnRowsInFlight; ++u) {
-      const int j = min(j0 + u * rpp + rr, nkeys - 1);
-      vv[u] = *reinterpret_cast<const uint4 *>(vbase + (size_t)j * hd);
-    }
-    attn_pv(vv, j0, nkeys, rpp, rr, s_p, acc);
-  }
-  float4 *sa = reinterpret_cast<float4 *>(s_acc + rr * hd + sub * 8);
-  sa[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-  sa[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
-  __syncthreads();
-  for (int d = threadIdx.x; d < hd; d += kAttnThreads) {
-    float o = 0.0f;
-    for (int r = 0; r < rpp; ++r) o += s_acc[r * hd + d];
-    out[((size_t)t * nq + h) * hd + d] = f32_to_bf16(o);
   }
 }
 
@@ -675,29 +516,6 @@ extern "C" int moe_rope_kv_bf16(const void *qkv, int64_t T, int32_t n_q_heads, i
                      (hipStream_t)stream, (const uint16_t *)qkv, n_q_heads, n_kv_heads, head_dim,
                      (const float *)inv_freq_f32, (const int32_t *)pos0_i32, max_seq,
                      (uint16_t *)q_out, (uint16_t *)k_cache, (uint16_t *)v_cache);
-  MOE_LAUNCH_CHECK();
-  return MOE_STATUS_OK;
-}
-
-extern "C" int moe_attention_bf16(const void *q, const void *k_cache, const void *v_cache, int64_t T,
-                                  int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
-                                  const void *pos0_i32, int64_t max_seq, float scaling, void *out,
-                                  void *stream) {
-  MOE_REQUIRE(T >= 0 && n_q_heads > 0 && n_kv_heads > 0 && n_q_heads % n_kv_heads == 0,
-              "query heads must be a multiple of the KV heads");
-  MOE_REQUIRE(head_dim > 0 && head_dim <= moe::kAttnMaxHeadDim && moe::kAttnThreads % head_dim == 0 &&
-                  head_dim % 8 == 0,
-              "head dim must divide %d and be a multiple of 8 (got %d)", moe::kAttnThreads, head_dim);
-  MOE_REQUIRE(max_seq > 0 && max_seq <= moe::kAttnMaxKeys, "max_seq must be in [1, %d]",
-              moe::kAttnMaxKeys);
-  if (T == 0) return MOE_STATUS_OK;
-  MOE_REQUIRE(q && k_cache && v_cache && pos0_i32 && out, "null pointer");
-  MOE_REQUIRE(((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0,
-              "q and the KV cache must be 16-byte aligned");
-  hipLaunchKernelGGL(moe::attention_kernel, dim3((unsigned)n_q_heads, (unsigned)T),
-                     dim3(moe::kAttnThreads), 0, (hipStream_t)stream, (const uint16_t *)q,
-                     (const uint16_t *)k_cache, (const uint16_t *)v_cache, n_q_heads, n_kv_heads,
-                     head_dim, (const int32_t *)pos0_i32, max_seq, scaling, (uint16_t *)out);
   MOE_LAUNCH_CHECK();
   return MOE_STATUS_OK;
 }

@@ -12,7 +12,6 @@ namespace {
 constexpr int kNormThreads = 256;
 constexpr int kNormMaxChunks = 8;  // 8-value chunks per thread: H <= 16384
 
-__device__ __forceinline__ float bf16r(float v) { return bf16_to_f32(f32_to_bf16(v)); }
 
 // Workgroup barrier that orders LDS only: a workgroup fence on all address spaces would
 // also wait for the wave's outstanding global loads (s_waitcnt vmcnt(0)), which in the

@@ -140,6 +140,13 @@ class NativeDecoder:
         self.moe = moe if moe is not None else self._moe_resident
         self._resident = moe is None
         self._moe_bufs = {}
+        # Attention workspace of every pass length (at most 20 MB), its counters zero between
+        # calls; never replaced, as captured steps hold its address.
+        n = 0
+        if self.dev.type == "cuda":
+            n = self.lib.moe_attention_workspace_bytes(self.max_seq, s.n_heads, s.n_kv_heads,
+                                                       s.head_dim, self.max_seq)
+        self._attn_ws = torch.zeros((n,), dtype=torch.uint8, device=self.dev) if n > 0 else None
         self._sb = None  # single-token step buffers
 
     # ------------------------------------------------------------------ pieces
@@ -164,6 +171,15 @@ class NativeDecoder:
             self._stream()), "add_rmsnorm")
         return out
 
+    def _attend(self, q, kc, vc, T: int, out) -> None:
+        """Attention of T query rows against a layer's cache, with the decoder's workspace (a
+        decoder runs one pass at a time, as its cache and position do)."""
+        s, ws = self.s, self._attn_ws
+        _lib.check(self.lib.moe_attention_ws_bf16(
+            q.data_ptr(), kc.data_ptr(), vc.data_ptr(), T, s.n_heads, s.n_kv_heads, s.head_dim,
+            self.pos.data_ptr(), self.max_seq, self.scaling, out.data_ptr(),
+            None if ws is None else ws.data_ptr(), 0 if ws is None else ws.numel(), self._stream()), "attention")
+
     def _attention(self, l: int, x1: torch.Tensor) -> torch.Tensor:
         s, T = self.s, x1.shape[0]
         qkv = self._linear(self.w.layers[l].qkv, x1)
@@ -174,10 +190,7 @@ class NativeDecoder:
                                              self.max_seq, q.data_ptr(), kc.data_ptr(), vc.data_ptr(),
                                              self._stream()), "rope_kv")
         a = torch.empty_like(q)
-        _lib.check(self.lib.moe_attention_bf16(q.data_ptr(), kc.data_ptr(), vc.data_ptr(), T,
-                                               s.n_heads, s.n_kv_heads, s.head_dim,
-                                               self.pos.data_ptr(), self.max_seq, self.scaling,
-                                               a.data_ptr(), self._stream()), "attention")
+        self._attend(q, kc, vc, T, a)
         return self._linear(self.w.layers[l].o_proj, a)
 
     def _moe_resident(self, l: int, x: torch.Tensor) -> torch.Tensor:
@@ -292,9 +305,7 @@ class NativeDecoder:
                 s.rms_eps, H, nq, nkv, hd, self.inv_freq.data_ptr(), self.pos.data_ptr(),
                 self.max_seq, b["h"].data_ptr(), b["q"].data_ptr(), kc.data_ptr(), vc.data_ptr(),
                 st), "qkv_rope")
-            _lib.check(lib.moe_attention_bf16(b["q"].data_ptr(), kc.data_ptr(), vc.data_ptr(), 1,
-                                              nq, nkv, hd, self.pos.data_ptr(), self.max_seq,
-                                              self.scaling, b["a"].data_ptr(), st), "attention")
+            self._attend(b["q"], kc, vc, 1, b["a"])
             _lib.check(lib.moe_gemv_bf16(lw.o_proj.data_ptr(), b["a"].data_ptr(), 1, H, nq * hd,
                                          b["y"].data_ptr(), st), "o_proj")
             if fused_moe:

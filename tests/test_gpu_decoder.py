@@ -116,6 +116,97 @@ def test_attention(cuda_device, T, p0, max_seq, hd):
     assert rel_l2(out.cpu(), want) < 4e-3
 
 
+def _attend(q, kc, vc, p0, ws):
+    """moe_attention_ws_bf16 (moe_attention_bf16 with ws None) of q [T, nq, hd] on the GPU."""
+    from moeinfra_amd import _lib
+
+    (T, nq, hd), (nkv, max_seq, _) = q.shape, kc.shape
+    out = torch.empty((T, nq * hd), dtype=torch.bfloat16, device=q.device)
+    pos = torch.tensor([p0], dtype=torch.int32, device=q.device)
+    args = (q.data_ptr(), kc.data_ptr(), vc.data_ptr(), T, nq, nkv, hd, pos.data_ptr(), max_seq,
+            hd ** -0.5, out.data_ptr())
+    st = torch.cuda.current_stream().cuda_stream
+    if ws is None:
+        _lib.check(_lib.lib().moe_attention_bf16(*args, st), "attention")
+    else:
+        _lib.check(_lib.lib().moe_attention_ws_bf16(*args, ws.data_ptr(), ws.numel(), st), "attention")
+    return out
+
+
+def _attend_ref(q, k, v, p0):
+    """Eager attention in fp32 with the bf16 roundings of the bf16 module, one query at a time
+    over the keys that it sees."""
+    T, nq, hd = q.shape
+    grp = nq // k.shape[0]
+    out = torch.empty((T, nq, hd))
+    for t in range(T):
+        K = k[:, :p0 + t + 1].float().repeat_interleave(grp, dim=0)
+        V = v[:, :p0 + t + 1].float().repeat_interleave(grp, dim=0)
+        sc = torch.einsum("hd,hkd->hk", q[t].float(), K).to(torch.bfloat16)
+        sc = (sc.float() * hd ** -0.5).to(torch.bfloat16).float()
+        p = torch.softmax(sc, dim=-1).to(torch.bfloat16).float()
+        out[t] = torch.einsum("hk,hkd->hd", p, V)
+    return out.reshape(T, -1)
+
+
+# Above 8 tokens the matrix form: row tiles of 128 (token, head of the group) rows, key tiles
+# of 64 keys, taken in pairs.  Up to 8 tokens a row's keys are shared between workgroups above
+# 384 of them.
+@pytest.mark.parametrize("T,p0,max_seq,nq,nkv,hd", [
+    (17, 0, 64, 4, 4, 128), (18, 46, 64, 8, 2, 64), (2, 0, 64, 4, 4, 128), (9, 50, 64, 8, 2, 64), (8, 380, 400, 8, 2, 64), (33, 95, 128, 32, 8, 128), (32, 128, 256, 4, 1, 128),
+    (129, 0, 256, 2, 2, 64), (65, 127, 200, 6, 2, 128), (17, 700, 1024, 8, 8, 64),
+    (5, 2500, 4096, 32, 8, 128), (40, 1000, 2048, 7, 1, 128),
+    (1, 383, 4096, 32, 8, 128), (1, 384, 4096, 32, 8, 128), (1, 640, 1000, 6, 3, 64),
+    (1, 8191, 8192, 8, 8, 256), (1, 2900, 4096, 8, 8, 128)])
+def test_attention_forms(cuda_device, T, p0, max_seq, nq, nkv, hd):
+    """Matrix form and shared keys: against the module's arithmetic, with cache rows past the
+    last key NaN; the workspace's counters return to zero, a second call repeats the bits."""
+    from moeinfra_amd import _lib
+
+    S = p0 + T
+    q, k, v = _bf16((T, nq, hd), 5), _bf16((nkv, S, hd), 6), _bf16((nkv, S, hd), 7)
+    kc = torch.full((nkv, max_seq, hd), float("nan"), dtype=torch.bfloat16)
+    vc = kc.clone()
+    kc[:, :S], vc[:, :S] = k, v
+    qd, kd, vd = q.to(cuda_device), kc.to(cuda_device), vc.to(cuda_device)
+    n = _lib.lib().moe_attention_workspace_bytes(T, nq, nkv, hd, max_seq)
+    ws = torch.zeros((max(n, 16),), dtype=torch.uint8, device=cuda_device)
+    want = _attend_ref(q, k, v, p0)
+    got = _attend(qd, kd, vd, p0, ws)
+    # As test_attention: bf16 rounding of the probabilities and of the output, 2^-9 each.
+    assert rel_l2(got.cpu(), want) < 4e-3
+    assert rel_l2(_attend(qd, kd, vd, p0, None).cpu(), want) < 4e-3
+    assert not ws[:4096].any()
+    assert torch.equal(_attend(qd, kd, vd, p0, ws), got)
+
+
+@pytest.mark.parametrize("T,p0,hd", [(40, 70, 128), (130, 0, 64), (20, 1500, 128), (6, 1500, 128)])
+def test_attention_nonfinite_values(cuda_device, T, p0, hd):
+    """An infinity or NaN in a V row reaches the queries that see the row and no others."""
+    from moeinfra_amd import _lib
+
+    nq, nkv, max_seq, S = 8, 2, 2048, p0 + T
+    q, k, v = _bf16((T, nq, hd), 15), _bf16((nkv, S, hd), 16), _bf16((nkv, S, hd), 17)
+    clean = v.clone()
+    bad = p0 + T // 2
+    v[0, bad, 3], v[1, bad + 1, hd - 1] = float("inf"), float("nan")
+    kc = torch.zeros((nkv, max_seq, hd), dtype=torch.bfloat16)
+    vc = kc.clone()
+    kc[:, :S], vc[:, :S] = k, v
+    qd, kd, vd = q.to(cuda_device), kc.to(cuda_device), vc.to(cuda_device)
+    n = _lib.lib().moe_attention_workspace_bytes(T, nq, nkv, hd, max_seq)
+    ws = torch.zeros((max(n, 16),), dtype=torch.uint8, device=cuda_device)
+    want = _attend_ref(q, k, clean, p0).reshape(T, nq, hd)
+    for w in (None, ws):
+        got = _attend(qd, kd, vd, p0, w).cpu().float().reshape(T, nq, hd)
+        t = torch.arange(T) + p0
+        hit = torch.zeros((T, nq, hd), dtype=torch.bool)
+        hit[t >= bad, :nq // 2, 3] = True
+        hit[t >= bad + 1, nq // 2:, hd - 1] = True
+        assert not torch.isfinite(got[hit]).any() and torch.isfinite(got[~hit]).all()
+        assert rel_l2(got.masked_fill(hit, 0.0), want.masked_fill(hit, 0.0)) < 4e-3
+
+
 @pytest.mark.parametrize("T,N,K", [(1, 6144, 4096), (1, 4096, 4096), (1, 1000, 512), (4, 515, 1024)])
 def test_gemv(cuda_device, T, N, K):
     from moeinfra_amd import _lib
