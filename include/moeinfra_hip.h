@@ -101,6 +101,12 @@ int moe_nf4_expand_absmax(const void *absmax_u8, const void *absmax2_f32, const 
 int moe_nf4_quantize_bf16(const void *w_bf16, int64_t numel, int32_t blocksize,
                           const void *code16, void *packed_out, void *absmax_out, void *stream);
 
+/* The same, also copying the codebook to code_out (fp32[16], may be null): the state of one
+ * weight in one launch. */
+int moe_nf4_quantize_state_bf16(const void *w_bf16, int64_t numel, int32_t blocksize,
+                                const void *code16, void *packed_out, void *absmax_out,
+                                void *code_out, void *stream);
+
 /* ---------------------------------------------------------------- K2: router
  * logits = bf16(x . gate^T); p = softmax(float(logits) [+ bias]); (w, idx) = top-k(p)
  * in descending order (ties: lower expert index first); w /= sum(w).

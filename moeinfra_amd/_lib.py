@@ -43,6 +43,7 @@ SIGNATURES = {
     "moe_wait_timeouts": ([ctypes.POINTER(_i64), _i32], ctypes.c_int),
     "moe_nf4_dequant_bf16": ([_vp, _vp, _vp, _vp, _i64, _i32, _vp], ctypes.c_int),
     "moe_nf4_quantize_bf16": ([_vp, _i64, _i32, _vp, _vp, _vp, _vp], ctypes.c_int),
+    "moe_nf4_quantize_state_bf16": ([_vp, _i64, _i32, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),
     "moe_router_topk": ([_vp, _vp, _vp, _i64, _i32, _i32, _i32, _vp, _vp, _vp, _vp, _vp],
                         ctypes.c_int),
     "moe_permute": ([_vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _vp, _vp], ctypes.c_int),

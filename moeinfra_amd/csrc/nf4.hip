@@ -65,61 +65,130 @@ constexpr int kQuantThreads = 256;
 
 // Blocksize-64 quantisation, eight lanes per block: lane l of a wave loads the 8 bf16 values
 // at 8*l of the wave's 512-value chunk (one contiguous 1 KB load per wave), the block's
-// absmax is the max over its 8 lanes (xor shuffles), and each lane packs its 8 values into
+// absmax is the max over its 8 lanes (DPP moves), and each lane packs its 8 values into
 // 4 bytes (one contiguous 256-byte store per wave).  Same arithmetic as the per-block kernel
-// below: q = number of codebook midpoints strictly below w * (1 / absmax), in fp32.
+// below: q = number of codebook midpoints strictly below y = w * (1 / absmax), in fp32.
+//
+// Bound: 2.56 bytes a value of HBM (31 us at the copy rate for a 14336 x 4096 projection).
+// Comparing y with all 15 midpoints is 30 VALU operations a value and took 72 us; the count
+// now comes from a table of 64 equal bins over [-1, 1].  A bin index is monotone in y, so
+// midpoints in lower bins are below y and those in higher bins are not; a bin holds at most
+// one midpoint of a codebook like NF4's (their distance is at least 2.5 bins), against which
+// one comparison decides: 36 us
+// (4.1 TB/s; 48 us while every thread built eight table entries and no load ran ahead).  The
+// entry {midpoint, count below the bin} has 32 replicas
+// (conflict-free ds_read_b64).  A codebook with two midpoints in a bin compares with all 15.
 constexpr int kQuant64Chunk = 512;
+constexpr int kQuantBins = 64;
+constexpr int kQuantReps = 32;
+
+// Bin of y: NaN and anything below -1 in the first, anything above 1 in the last.
+__device__ __forceinline__ uint32_t quant_bin(float y) {
+  const float t = fmaf(y, 0.5f * kQuantBins, 0.5f * kQuantBins);
+  return (uint32_t)fminf(fmaxf(t, 0.0f), (float)(kQuantBins - 1));
+}
+
+template <bool BINS>
+__device__ __forceinline__ uint32_t quant8(const u32x4 raw, float r, const float *mid, const float2 *bins,
+                                           uint32_t rep) {
+  uint32_t out = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float y = ((i & 1) ? bf16hi_to_f32(raw[i >> 1]) : bf16lo_to_f32(raw[i >> 1])) * r;
+    uint32_t q = 0;
+    if constexpr (BINS) {
+      const float2 e = bins[quant_bin(y) * kQuantReps + rep];
+      q = __builtin_bit_cast(uint32_t, e.y) + (y > e.x ? 1u : 0u);
+    } else {
+      for (int m = 0; m < 15; ++m) q += y > mid[m] ? 1u : 0u;
+    }
+    // value 2j in the high nibble of byte j
+    out |= q << (8 * (i >> 1) + ((i & 1) ? 0 : 4));
+  }
+  return out;
+}
+
+template <bool BINS>
+__device__ __forceinline__ void quant64_chunks(const uint16_t *w, int64_t nchunk, uint8_t *packed, float *absmax,
+                                               const float *mid, const float2 *bins) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const uint32_t rep = threadIdx.x & (kQuantReps - 1);
+  const int64_t waves = (int64_t)gridDim.x * (kQuantThreads / kWave);
+  const int64_t c0 = (int64_t)blockIdx.x * (kQuantThreads / kWave) + (threadIdx.x >> 6);
+  // Two chunks per step, the next step's loads in flight under this one's arithmetic (past
+  // the end: the last chunk again, unused).
+  auto load = [&](int64_t c) {
+    const uint4 v = ld_stream16(w + (c < nchunk ? c : nchunk - 1) * kQuant64Chunk + 8 * lane);
+    return u32x4{v.x, v.y, v.z, v.w};
+  };
+  u32x4 next[2] = {load(c0), load(c0 + waves)};
+  for (int64_t c = c0; c < nchunk; c += 2 * waves) {
+    const u32x4 raw[2] = {next[0], next[1]};
+    next[0] = load(c + 2 * waves);
+    next[1] = load(c + 3 * waves);
+    float amax[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        amax[u] = fmaxf(amax[u], fabsf(bf16lo_to_f32(raw[u][i])));
+        amax[u] = fmaxf(amax[u], fabsf(bf16hi_to_f32(raw[u][i])));
+      }
+    lane_groups_reduce<true>(amax, 8);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      if (u == 1 && c + waves >= nchunk) break;
+      const int64_t v0 = (c + u * waves) * kQuant64Chunk + 8 * lane;
+      if ((lane & 7) == 0) absmax[v0 / 64] = amax[u];
+      const float r = amax[u] > 0.0f ? 1.0f / amax[u] : 0.0f;
+      *reinterpret_cast<uint32_t *>(packed + v0 / 2) = quant8<BINS>(raw[u], r, mid, bins, rep);
+    }
+  }
+}
 
 __global__ void __launch_bounds__(kQuantThreads)
 nf4_quantize64_kernel(const uint16_t *__restrict__ w, int64_t nchunk,
                       const float *__restrict__ code, uint8_t *__restrict__ packed,
-                      float *__restrict__ absmax) {
-  __shared__ float s_mid[16];
+                      float *__restrict__ absmax, float *__restrict__ code_out) {
+  __shared__ float s_mid[15];
+  __shared__ float2 s_bins[kQuantBins * kQuantReps];
   if (threadIdx.x < 15) s_mid[threadIdx.x] = (code[threadIdx.x] + code[threadIdx.x + 1]) * 0.5f;
+  if (code_out != nullptr && blockIdx.x == 0 && threadIdx.x < 16) code_out[threadIdx.x] = code[threadIdx.x];
   __syncthreads();
-  float mid[15];
-#pragma unroll
-  for (int m = 0; m < 15; ++m) mid[m] = s_mid[m];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int64_t waves = (int64_t)gridDim.x * (kQuantThreads / kWave);
-  for (int64_t c = (int64_t)blockIdx.x * (kQuantThreads / kWave) + (threadIdx.x >> 6); c < nchunk;
-       c += waves) {
-    const int64_t v0 = c * kQuant64Chunk + 8 * lane;
-    const u32x4 raw = *reinterpret_cast<const u32x4 *>(w + v0);
-    float x[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const uint32_t word = raw[i];
-      x[2 * i] = bf16lo_to_f32(word);
-      x[2 * i + 1] = bf16hi_to_f32(word);
+  // One thread per bin, then the replicas.
+  int crowded = 0;
+  if (threadIdx.x < kQuantBins) {
+    float thr = INFINITY;
+    uint32_t below = 0, in = 0;
+    for (int m = 0; m < 15; ++m) {
+      const float x = s_mid[m];
+      const uint32_t bm = quant_bin(x);
+      const bool number = x == x;  // nothing is above a NaN
+      below += number && bm < threadIdx.x ? 1u : 0u;
+      thr = number && bm == threadIdx.x ? x : thr;
+      in += number && bm == threadIdx.x ? 1u : 0u;
     }
-    float amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[i]));
-#pragma unroll
-    for (int off = 1; off < 8; off <<= 1) amax = fmaxf(amax, __shfl_xor(amax, off, kWave));
-    if ((lane & 7) == 0) absmax[v0 / 64] = amax;
-    const float r = amax > 0.0f ? 1.0f / amax : 0.0f;
-    uint32_t out = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float y = x[i] * r;
-      uint32_t q = 0;
-#pragma unroll
-      for (int m = 0; m < 15; ++m) q += y > mid[m] ? 1u : 0u;
-      // value 2j in the high nibble of byte j
-      out |= q << (8 * (i >> 1) + ((i & 1) ? 0 : 4));
-    }
-    *reinterpret_cast<uint32_t *>(packed + v0 / 2) = out;
+    crowded = in > 1u;
+    s_bins[threadIdx.x * kQuantReps] = make_float2(thr, __builtin_bit_cast(float, below));
   }
+  const bool general = __syncthreads_or(crowded) != 0;
+  for (int i = threadIdx.x; i < kQuantBins * kQuantReps; i += kQuantThreads)
+    if (i % kQuantReps != 0) s_bins[i] = s_bins[i / kQuantReps * kQuantReps];
+  __syncthreads();
+  // Uniform over the grid: every workgroup builds the same table.
+  if (general)
+    quant64_chunks<false>(w, nchunk, packed, absmax, s_mid, s_bins);
+  else
+    quant64_chunks<true>(w, nchunk, packed, absmax, s_mid, s_bins);
 }
 
 // One thread per quantisation block: any blocksize, partial last block.
 __global__ void __launch_bounds__(kQuantThreads)
 nf4_quantize_kernel(const uint16_t *__restrict__ w, int64_t numel, int32_t blocksize,
                     const float *__restrict__ code, uint8_t *__restrict__ packed,
-                    float *__restrict__ absmax) {
+                    float *__restrict__ absmax, float *__restrict__ code_out) {
   __shared__ float s_mid[15];
+  if (code_out != nullptr && blockIdx.x == 0 && threadIdx.x < 16) code_out[threadIdx.x] = code[threadIdx.x];
   if (threadIdx.x < 15) s_mid[threadIdx.x] = (code[threadIdx.x] + code[threadIdx.x + 1]) * 0.5f;
   __syncthreads();
   const int64_t nblocks = (numel + blocksize - 1) / blocksize;
@@ -209,6 +278,13 @@ extern "C" int moe_nf4_dequant_bf16(const void *packed, const void *absmax, cons
 extern "C" int moe_nf4_quantize_bf16(const void *w_bf16, int64_t numel, int32_t blocksize,
                                      const void *code16, void *packed_out, void *absmax_out,
                                      void *stream) {
+  return moe_nf4_quantize_state_bf16(w_bf16, numel, blocksize, code16, packed_out, absmax_out, nullptr,
+                                     stream);
+}
+
+extern "C" int moe_nf4_quantize_state_bf16(const void *w_bf16, int64_t numel, int32_t blocksize,
+                                           const void *code16, void *packed_out, void *absmax_out,
+                                           void *code_out, void *stream) {
   MOE_REQUIRE(numel >= 0 && numel % 2 == 0, "numel must be even and non-negative (got %lld)",
               (long long)numel);
   MOE_REQUIRE(blocksize >= 2 && blocksize <= 4096 && blocksize % 2 == 0,
@@ -223,7 +299,8 @@ extern "C" int moe_nf4_quantize_bf16(const void *w_bf16, int64_t numel, int32_t 
     blocks = blocks > cap ? cap : blocks;
     hipLaunchKernelGGL(moe::nf4_quantize64_kernel, dim3((unsigned)blocks), dim3(moe::kQuantThreads),
                        0, (hipStream_t)stream, (const uint16_t *)w_bf16, nchunk,
-                       (const float *)code16, (uint8_t *)packed_out, (float *)absmax_out);
+                       (const float *)code16, (uint8_t *)packed_out, (float *)absmax_out,
+                       (float *)code_out);
     MOE_LAUNCH_CHECK();
     return MOE_STATUS_OK;
   }
@@ -232,7 +309,8 @@ extern "C" int moe_nf4_quantize_bf16(const void *w_bf16, int64_t numel, int32_t 
   MOE_REQUIRE(grid <= 0x7fffffff, "numel too large");
   hipLaunchKernelGGL(moe::nf4_quantize_kernel, dim3((unsigned)grid), dim3(moe::kQuantThreads), 0,
                      (hipStream_t)stream, (const uint16_t *)w_bf16, numel, blocksize,
-                     (const float *)code16, (uint8_t *)packed_out, (float *)absmax_out);
+                     (const float *)code16, (uint8_t *)packed_out, (float *)absmax_out,
+                     (float *)code_out);
   MOE_LAUNCH_CHECK();
   return MOE_STATUS_OK;
 }

@@ -113,8 +113,8 @@ class NF4Linear(nn.Module):
         """Quantise the bf16 weight in place on its (GPU) device with the HIP quantiser."""
         if self.quantized:
             return self
-        packed, absmax, code = ops.nf4_quantize(self.weight.contiguous(), NF4_BLOCKSIZE)
-        self.quant_state = NF4QuantState(absmax=absmax, code=code.clone(),
+        packed, absmax, code = ops.nf4_quantize(self.weight.contiguous(), NF4_BLOCKSIZE, own_code=True)
+        self.quant_state = NF4QuantState(absmax=absmax, code=code,
                                           shape=torch.Size((self.out_features, self.in_features)))
         self.weight = packed
         return self

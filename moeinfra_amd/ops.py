@@ -101,8 +101,9 @@ def nf4_dequant(packed: torch.Tensor, absmax: torch.Tensor, code: torch.Tensor,
 
 # ----------------------------------------------------------------------------- K0
 def nf4_quantize(w: torch.Tensor, blocksize: int = NF4_BLOCKSIZE,
-                 code: Optional[torch.Tensor] = None):
-    """bf16 weight -> (packed uint8 [numel//2, 1], absmax fp32 [nblocks], code fp32 [16])."""
+                 code: Optional[torch.Tensor] = None, own_code: bool = False):
+    """bf16 weight -> (packed uint8 [numel//2, 1], absmax fp32 [nblocks], code fp32 [16]).
+    ``own_code``: the returned code is a new tensor that the launch fills, not the shared one."""
     dev = w.device
     _require_cuda(w, "weight")
     if w.dtype != torch.bfloat16:
@@ -116,9 +117,13 @@ def nf4_quantize(w: torch.Tensor, blocksize: int = NF4_BLOCKSIZE,
         raise ValueError("NF4 packing needs an even number of values")
     packed = torch.empty((numel // 2, 1), dtype=torch.uint8, device=dev)
     absmax = torch.empty(((numel + blocksize - 1) // blocksize,), dtype=torch.float32, device=dev)
-    check(lib().moe_nf4_quantize_bf16(w.data_ptr(), numel, blocksize, code.data_ptr(),
-                                      packed.data_ptr(), absmax.data_ptr(), _stream(dev)),
-          "nf4_quantize")
+    # (an empty weight launches nothing, so its code is copied)
+    mine = torch.empty_like(code) if own_code and numel else None
+    check(lib().moe_nf4_quantize_state_bf16(w.data_ptr(), numel, blocksize, code.data_ptr(),
+                                            packed.data_ptr(), absmax.data_ptr(), _ptr(mine),
+                                            _stream(dev)), "nf4_quantize")
+    if own_code:
+        return packed, absmax, code.clone() if mine is None else mine
     return packed, absmax, code
 
 

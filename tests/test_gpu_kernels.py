@@ -68,6 +68,42 @@ def test_quantize_bitexact(cuda_device, shape):
     np.testing.assert_array_equal(a_got.cpu().numpy(), a_want)
 
 
+@pytest.mark.parametrize("case", ["nf4", "crowded", "unsorted", "nan_code"])
+@pytest.mark.parametrize("chunks", [1, 2, 8192 + 3])
+def test_quantize_binned_is_general(cuda_device, case, chunks):
+    """The blocksize-64 kernel (midpoints counted through a table of bins) against the general
+    one (every midpoint compared), for any codebook and any weights: bit for bit."""
+    from moeinfra_amd import _lib, ops
+
+    code = torch.from_numpy(orc.NF4_CODE.copy())
+    if case == "crowded":          # two midpoints in one bin of 1/32
+        code[8] = 0.01
+    elif case == "unsorted":
+        code = code[torch.randperm(16, generator=torch.Generator().manual_seed(1))].contiguous()
+    elif case == "nan_code":
+        code[3], code[12] = float("nan"), float("inf")
+    code = code.to(cuda_device)
+    n = 512 * chunks
+    w = torch.randn((n,), generator=torch.Generator().manual_seed(chunks)).mul_(0.02)
+    w[64:128] = 0.0
+    w[128:192] *= 1e-38                                  # subnormal block, then special values
+    w[200], w[280], w[300], w[340] = float("nan"), float("inf"), float("-inf"), -0.0
+    w[384:448] = torch.linspace(-1, 1, 64)               # values on and next to bin edges
+    buf = torch.empty((n + 8,), dtype=torch.bfloat16, device=cuda_device)
+    buf[:n] = w.to(torch.bfloat16).to(cuda_device)
+    got = ops.nf4_quantize(buf[:n], code=code, own_code=True)
+    aligned = buf[:n].clone()
+    buf[1:n + 1] = aligned                               # 2-byte aligned: the general kernel
+    packed = torch.empty((n // 2,), dtype=torch.uint8, device=cuda_device)
+    absmax = torch.empty((n // 64,), dtype=torch.float32, device=cuda_device)
+    _lib.check(_lib.lib().moe_nf4_quantize_bf16(buf.data_ptr() + 2, n, 64, code.data_ptr(), packed.data_ptr(),
+                                                absmax.data_ptr(), torch.cuda.current_stream().cuda_stream), "q")
+    np.testing.assert_array_equal(got[0].cpu().numpy().reshape(-1), packed.cpu().numpy())
+    np.testing.assert_array_equal(got[1].cpu().numpy().view(np.uint32), absmax.cpu().numpy().view(np.uint32))
+    assert got[2].data_ptr() != code.data_ptr()
+    np.testing.assert_array_equal(got[2].cpu().numpy().view(np.uint32), code.cpu().numpy().view(np.uint32))
+
+
 # ------------------------------------------------------------------------------ K2
 @pytest.mark.parametrize("T,H,E,skew,k", [(1, 4096, 8, False, 2), (16, 1024, 8, False, 2),
                                           (40, 4096, 8, True, 2), (513, 4096, 8, False, 2),
