@@ -14,7 +14,9 @@ int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x,
                       int32_t k, int32_t H, int32_t F, const int32_t *counts,
                       const int32_t *offsets, const int32_t *perm_tok, const int32_t *active,
                       void *h_ws, void *ypart, int32_t nsplit, int64_t max_tokens_per_expert,
-                      int phases, hipStream_t stream, const FusedCombine *fused);
+                      int phases, hipStream_t stream, const FusedCombine *fused,
+                      uint8_t *planes);
+int layer_range_planes(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, int *cols);
 bool gemv4_supported(int64_t max_tokens_per_expert, int32_t H, int32_t F);
 bool route_small_supported(int64_t T, int32_t k);
 int launch_route_small(const void *x, const void *gate, const void *bias, int64_t T, int32_t H,
@@ -23,11 +25,11 @@ int launch_route_small(const void *x, const void *gate, const void *bias, int64_
                        void *zero_word, hipStream_t stream);
 int launch_combine(const void *ypart, int32_t nsplit, const void *weights, const void *idx_i32,
                    const void *slot_pos, int64_t T, int32_t k, int32_t H, void *out,
-                   hipStream_t stream);
+                   const uint8_t *planes, int cols, hipStream_t stream);
 int launch_identity_route(int64_t T, int32_t *counts, int32_t *offsets, int32_t *perm_tok,
                           int32_t *active, hipStream_t stream);
 int launch_reduce_splits(const float *ypart, int nsplit, int64_t numel, uint16_t *y,
-                         hipStream_t stream);
+                         const uint8_t *planes, int cols, hipStream_t stream);
 bool decode_layer_supported(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F);
 bool mid_layer_supported(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F);
 bool mid_group_supported(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F);
@@ -76,15 +78,23 @@ int64_t align_up(int64_t v) { return (v + kAlign - 1) / kAlign * kAlign; }
 // Byte offsets of the layer workspace regions.
 struct LayerWs {
   int64_t idx32, counts, offsets, perm_tok, slot_pos, active, counter, droute, h, ypart,
-      ypart_bytes, total;
+      ypart_bytes, pieces, total;
   int nsplit;
+  int cols;  // > 0: the down projection runs in ranges, `pieces` bytes per item of cols columns
 };
 
-// nsplit_override > 0 replaces the default number of down-projection ypart planes.
-LayerWs layer_ws(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, int nsplit_override = 0) {
+// one_plane: a single ypart plane instead of the default number.
+LayerWs layer_ws(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, bool one_plane = false) {
   LayerWs w{};
   const int64_t rows = T * k;
-  w.nsplit = nsplit_override > 0 ? nsplit_override : choose_nsplit(T, k, E, H, F);
+  int planes = choose_nsplit(T, k, E, H, F);
+  w.nsplit = one_plane ? 1 : planes;
+  const int ranges = one_plane ? 0 : layer_range_planes(T, k, E, H, F, &w.cols);
+  if (ranges > 0) {
+    w.nsplit = ranges;
+    planes = ranges > planes ? ranges : planes;
+  }
+  if (one_plane) planes = 1;
   int64_t o = 0;
   w.idx32 = o;    o = align_up(o + rows * 4);
   w.counts = o;   o = align_up(o + (int64_t)E * 4);
@@ -95,20 +105,23 @@ LayerWs layer_ws(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, int nspl
   w.counter = o;  o = align_up(o + 4);
   w.droute = o;   o = align_up(o + decode_route_bytes());
   w.h = o;        o = align_up(o + rows * (int64_t)F * 2);
-  w.ypart = o;    o = align_up(o + (int64_t)w.nsplit * rows * H * 4);
+  w.ypart = o;    o = align_up(o + (int64_t)planes * rows * H * 4);
   w.ypart_bytes = o - w.ypart;
+  w.pieces = o;   o = align_up(o + (w.cols > 0 ? rows * (H / w.cols) : 0));
   w.total = o;
   return w;
 }
 
 struct ExpertWs {
-  int64_t counts, offsets, perm_tok, active, h, ypart, total;
+  int64_t counts, offsets, perm_tok, active, h, ypart, pieces, total;
   int nsplit;
+  int cols;
 };
 
 ExpertWs expert_ws(int64_t T, int32_t H, int32_t F) {
   ExpertWs w{};
-  w.nsplit = choose_nsplit(T, 1, 1, H, F);
+  const int ranges = layer_range_planes(T, 1, 1, H, F, &w.cols);
+  w.nsplit = ranges > 0 ? ranges : choose_nsplit(T, 1, 1, H, F);
   int64_t o = 0;
   w.counts = o;   o = align_up(o + 4);
   w.offsets = o;  o = align_up(o + 8);
@@ -116,6 +129,7 @@ ExpertWs expert_ws(int64_t T, int32_t H, int32_t F) {
   w.active = o;   o = align_up(o + 8);
   w.h = o;        o = align_up(o + T * (int64_t)F * 2);
   w.ypart = o;    o = align_up(o + (int64_t)w.nsplit * T * H * 4);
+  w.pieces = o;   o = align_up(o + (w.cols > 0 ? T * (H / w.cols) : 0));
   w.total = o;
   return w;
 }
@@ -177,11 +191,11 @@ int layer_forward(const moe_nf4_expert_t *experts, int32_t E, const void *gate_b
                   const void *bias_f32, const void *x_bf16, int64_t T, int32_t H, int32_t F,
                   int32_t k, void *out_bf16, void *logits_bf16, void *weights_f32, void *idx_i64,
                   void *workspace, int64_t workspace_bytes, hipStream_t s, hipEvent_t *ev,
-                  int nsplit_override = 0) {
+                  bool one_plane = false) {
   MOE_REQUIRE(T >= 0 && k >= 1 && E >= 1 && H >= 1 && F >= 1, "bad sizes");
   if (T == 0) return MOE_STATUS_OK;
   MOE_REQUIRE(out_bf16 && weights_f32 && idx_i64, "null output pointer");
-  const LayerWs w = layer_ws(T, k, E, H, F, nsplit_override);
+  const LayerWs w = layer_ws(T, k, E, H, F, one_plane);
   MOE_REQUIRE(workspace != nullptr && workspace_bytes >= w.total,
               "workspace too small: need %lld bytes, got %lld", (long long)w.total,
               (long long)workspace_bytes);
@@ -193,6 +207,7 @@ int layer_forward(const moe_nf4_expert_t *experts, int32_t E, const void *gate_b
   int32_t *slot_pos = at<int32_t>(workspace, w.slot_pos);
   int32_t *active = at<int32_t>(workspace, w.active);
   uint32_t *counter = at<uint32_t>(workspace, w.counter);
+  uint8_t *pieces = w.cols > 0 ? at<uint8_t>(workspace, w.pieces) : nullptr;
   if (decode_layer_supported(T, k, E, H, F))
     return launch_decode_layer(experts, E, gate_bf16, bias_f32, x_bf16, T, H, F, k, out_bf16,
                                logits_bf16, weights_f32, idx_i64, at<void>(workspace, w.droute),
@@ -248,7 +263,7 @@ int layer_forward(const moe_nf4_expert_t *experts, int32_t E, const void *gate_b
     if (ev) MOE_HIP_CHECK(hipEventRecord(ev[1], s));
     rc = launch_expert_ffn(experts, E, x_bf16, T, k, H, F, counts, offsets, perm_tok, active,
                            at<void>(workspace, w.h), at<void>(workspace, w.ypart), w.nsplit, T, 1,
-                           s, nullptr);
+                           s, nullptr, pieces);
     if (rc != MOE_STATUS_OK) return rc;
   }
   if (ev) MOE_HIP_CHECK(hipEventRecord(ev[2], s));
@@ -260,11 +275,11 @@ int layer_forward(const moe_nf4_expert_t *experts, int32_t E, const void *gate_b
                         (int)T, k};
   rc = launch_expert_ffn(experts, E, nullptr, T, k, H, F, counts, offsets, perm_tok, active,
                          at<void>(workspace, w.h), at<void>(workspace, w.ypart), w.nsplit, T, 2,
-                         s, fuse ? &fc : nullptr);
+                         s, fuse ? &fc : nullptr, pieces);
   if (rc != MOE_STATUS_OK) return rc;
   if (!fuse) {
     rc = launch_combine(at<void>(workspace, w.ypart), w.nsplit, weights_f32, idx32, slot_pos, T,
-                        k, H, out_bf16, s);
+                        k, H, out_bf16, pieces, w.cols, s);
     if (rc != MOE_STATUS_OK) return rc;
   }
   if (ev) MOE_HIP_CHECK(hipEventRecord(ev[3], s));
@@ -324,16 +339,17 @@ extern "C" int moe_expert_swiglu_nf4(const moe_nf4_expert_t *expert, const void 
                                       moe::at<int32_t>(workspace, w.perm_tok),
                                       moe::at<int32_t>(workspace, w.active), s);
   if (rc != MOE_STATUS_OK) return rc;
+  uint8_t *pieces = w.cols > 0 ? moe::at<uint8_t>(workspace, w.pieces) : nullptr;
   rc = moe::launch_expert_ffn(expert, 1, x_bf16, T, 1, H, F,
                               moe::at<int32_t>(workspace, w.counts),
                               moe::at<int32_t>(workspace, w.offsets),
                               moe::at<int32_t>(workspace, w.perm_tok),
                               moe::at<int32_t>(workspace, w.active),
                               moe::at<void>(workspace, w.h), moe::at<void>(workspace, w.ypart),
-                              w.nsplit, T, 3, s, nullptr);
+                              w.nsplit, T, 3, s, nullptr, pieces);
   if (rc != MOE_STATUS_OK) return rc;
   return moe::launch_reduce_splits(moe::at<float>(workspace, w.ypart), w.nsplit, T * (int64_t)H,
-                                   (uint16_t *)y_bf16, s);
+                                   (uint16_t *)y_bf16, pieces, w.cols, s);
 }
 
 namespace {
@@ -429,14 +445,12 @@ extern "C" int moe_layer_forward_nf4_noalloc(const moe_nf4_expert_t *experts, in
                                              void *idx_i64, void *stream) {
   MOE_REQUIRE(T >= 0 && k >= 1 && E >= 1 && H >= 1 && F >= 1, "bad sizes");
   if (T == 0) return MOE_STATUS_OK;
-  // When the default layout (down-projection K splits over several ypart planes) does not
-  // fit the scratch, one plane: the same results, fewer workgroups on the down projection.
-  int nsplit = 0;
+  // When the default layout (pieces or K splits of the down projection over several ypart
+  // planes) does not fit the scratch, one plane: the same results up to the order of fp32
+  // sums, fewer workgroups on the down projection.
   int64_t need = moe::layer_ws(T, k, E, H, F).total;
-  if (need > MOE_NOALLOC_SCRATCH_BYTES) {
-    nsplit = 1;
-    need = moe::layer_ws(T, k, E, H, F, 1).total;
-  }
+  const bool one_plane = need > MOE_NOALLOC_SCRATCH_BYTES;
+  if (one_plane) need = moe::layer_ws(T, k, E, H, F, true).total;
   MOE_REQUIRE(need <= MOE_NOALLOC_SCRATCH_BYTES,
               "layer needs %lld bytes of workspace, above the %lld-byte static scratch; call "
               "moe_layer_forward_nf4 with a workspace",
@@ -446,5 +460,5 @@ extern "C" int moe_layer_forward_nf4_noalloc(const moe_nf4_expert_t *experts, in
   if (rc != MOE_STATUS_OK) return rc;
   return moe::layer_forward(experts, E, gate_bf16, bias_f32, x_bf16, T, H, F, k, out_bf16,
                             logits_bf16, weights_f32, idx_i64, ws, MOE_NOALLOC_SCRATCH_BYTES,
-                            (hipStream_t)stream, nullptr, nsplit);
+                            (hipStream_t)stream, nullptr, one_plane);
 }

@@ -329,7 +329,8 @@ constexpr int kCombineCols = kCombineThreads * 4;
 __global__ void __launch_bounds__(kCombineThreads)
 combine_kernel(const float *__restrict__ ypart, int nsplit, int64_t rows_total,
                const float *__restrict__ wts, const int32_t *__restrict__ idx,
-               const int32_t *__restrict__ slot_pos, int k, int H, uint16_t *__restrict__ out) {
+               const int32_t *__restrict__ slot_pos, int k, int H, uint16_t *__restrict__ out,
+               const uint8_t *__restrict__ planes, int cols) {
   const int64_t t = blockIdx.x;
   const int c = blockIdx.y * kCombineCols + threadIdx.x * 4;
   if (c >= H) return;
@@ -357,8 +358,10 @@ combine_kernel(const float *__restrict__ ypart, int nsplit, int64_t rows_total,
     if (pos < 0 || pos >= rows_total) continue;
     const float w = wts[t * k + j];
     float4 y = *reinterpret_cast<const float4 *>(ypart + (size_t)pos * H + c);
+    // Planes of this row's item: all, or as many as it has pieces (cols output columns each).
+    const int np = planes != nullptr ? planes[(size_t)pos * (H / cols) + c / cols] : nsplit;
 #pragma unroll 4
-    for (int s = 1; s < nsplit; ++s) {
+    for (int s = 1; s < np; ++s) {
       const float4 v = *reinterpret_cast<const float4 *>(ypart + s * split_stride + (size_t)pos * H + c);
       y.x += v.x;
       y.y += v.y;
@@ -390,11 +393,15 @@ __global__ void identity_route_kernel(int64_t T, int32_t *counts, int32_t *offse
 }
 
 __global__ void reduce_splits_kernel(const float *__restrict__ ypart, int nsplit, int64_t numel,
-                                     uint16_t *__restrict__ y) {
+                                     uint16_t *__restrict__ y, const uint8_t *__restrict__ planes,
+                                     int cols) {
   const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (i >= numel) return;
   float4 acc = *reinterpret_cast<const float4 *>(ypart + i);
-  for (int s = 1; s < nsplit; ++s) {
+  // Row i / H's items follow each other in `planes`, cols columns each (H a multiple).
+  const int np = planes != nullptr ? planes[i / cols] : nsplit;
+#pragma unroll 4
+  for (int s = 1; s < np; ++s) {
     const float4 v = *reinterpret_cast<const float4 *>(ypart + (size_t)s * numel + i);
     acc.x += v.x;
     acc.y += v.y;
@@ -438,7 +445,11 @@ bool expert_gemm_rows_ok(int64_t T, int64_t rows_total, int32_t H, int32_t F);
 int expert_gemm_splits(int64_t rows, int64_t active, int32_t H, int32_t F);
 int launch_expert_gemm(const void *tab, const void *x, int64_t T, int64_t rows_total,
                        int64_t active_max, int32_t H, int32_t F, const void *route, void *h_ws,
-                       void *ypart, int32_t nsplit, int phases, hipStream_t stream);
+                       void *ypart, int32_t nsplit, int phases, uint8_t *planes,
+                       hipStream_t stream);
+int expert_gemm_planes(int64_t rows, int64_t active, int32_t H, int32_t F);
+bool expert_gemm_ranges_ok(int64_t rows, int64_t active, int32_t H, int32_t F);
+int expert_gemm_down_cols(int64_t rows, int64_t active);
 // Average routed rows per expert from which a layer uses the batched GEMM.
 constexpr int64_t kGemmMinRowsPerExpert = 32;
 
@@ -480,6 +491,19 @@ int choose_nsplit(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F) {
   return midbatch_splits(active_max, H, F);
 }
 
+// ypart planes of a layer (T tokens, k slots, E experts) whose down projection runs in ranges
+// on the batched GEMM, and its output columns per item; 0 for other layers.
+int layer_range_planes(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, int *cols) {
+  const int64_t rows = T * k;
+  const int64_t active_max = rows < E ? rows : E;
+  if (T <= 0 || gemv4_supported(T, H, F) || mid_down_supported(T, k, E, H, F) ||
+      rows < kGemmMinRowsPerExpert * active_max || !expert_gemm_supported(H, F) ||
+      !expert_gemm_rows_ok(T, rows, H, F) || !expert_gemm_ranges_ok(rows, active_max, H, F))
+    return 0;
+  *cols = expert_gemm_down_cols(rows, active_max);
+  return expert_gemm_planes(rows, active_max, H, F);
+}
+
 bool mid_layer_supported(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F);
 
 // Gate/up of a mid-size layer with the routing and grouping in the same launch (every
@@ -512,7 +536,8 @@ int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x,
                       int32_t k, int32_t H, int32_t F, const int32_t *counts,
                       const int32_t *offsets, const int32_t *perm_tok, const int32_t *active,
                       void *h_ws, void *ypart, int32_t nsplit, int64_t max_tokens_per_expert,
-                      int phases, hipStream_t stream, const FusedCombine *fused) {
+                      int phases, hipStream_t stream, const FusedCombine *fused,
+                      uint8_t *planes) {
   MOE_REQUIRE(E >= 1 && E <= MOE_MAX_EXPERTS, "num_experts must be in [1, %d]", MOE_MAX_EXPERTS);
   MOE_REQUIRE(H > 0 && H % 256 == 0, "hidden size must be a positive multiple of 256 (got %d)", H);
   MOE_REQUIRE(F > 0 && F % 256 == 0, "FFN size must be a positive multiple of 256 (got %d)", F);
@@ -561,10 +586,10 @@ int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x,
   // Many tokens per expert on average: the LDS-staged GEMM streams each weight tile once per
   // 128 tokens (the per-tile kernels below re-stream it every 16 or 32 tokens).
   if (fused == nullptr && rows_total >= kGemmMinRowsPerExpert * active_max &&
-      expert_gemm_supported(H, F) && expert_gemm_splits_ok(F, nsplit) &&
+      expert_gemm_supported(H, F) && (planes != nullptr || expert_gemm_splits_ok(F, nsplit)) &&
       expert_gemm_rows_ok(T, rows_total, H, F))
     return launch_expert_gemm(&tab, x, T, rows_total, active_max, H, F, &rt, h_ws, ypart, nsplit,
-                              phases, stream);
+                              phases, planes, stream);
   // Fewer: the mid-batch kernels stream each weight tile once per 32 tokens of its expert
   // (32x32x16 MFMA, 16-byte weight loads): the streamed form (whole-K waves, activations
   // through LDS, `nsplit` K splits of the down projection) where the shape allows, else the
@@ -605,7 +630,7 @@ int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x,
 
 int launch_combine(const void *ypart, int32_t nsplit, const void *weights, const void *idx_i32,
                    const void *slot_pos, int64_t T, int32_t k, int32_t H, void *out,
-                   hipStream_t stream) {
+                   const uint8_t *planes, int cols, hipStream_t stream) {
   MOE_REQUIRE(T >= 0 && T <= 0x7fffffff, "T out of range");
   MOE_REQUIRE(k >= 1 && k <= MOE_MAX_TOPK, "top-k must be in [1, %d]", MOE_MAX_TOPK);
   MOE_REQUIRE(H > 0 && H % 4 == 0, "hidden size must be a positive multiple of 4");
@@ -617,7 +642,8 @@ int launch_combine(const void *ypart, int32_t nsplit, const void *weights, const
   const unsigned cgrid = (unsigned)((H + kCombineCols - 1) / kCombineCols);
   hipLaunchKernelGGL(combine_kernel, dim3((unsigned)T, cgrid), dim3(kCombineThreads), 0, stream,
                      (const float *)ypart, nsplit, T * k, (const float *)weights,
-                     (const int32_t *)idx_i32, (const int32_t *)slot_pos, k, H, (uint16_t *)out);
+                     (const int32_t *)idx_i32, (const int32_t *)slot_pos, k, H, (uint16_t *)out,
+                     planes, cols);
   MOE_LAUNCH_CHECK();
   return MOE_STATUS_OK;
 }
@@ -632,11 +658,11 @@ int launch_identity_route(int64_t T, int32_t *counts, int32_t *offsets, int32_t 
 }
 
 int launch_reduce_splits(const float *ypart, int nsplit, int64_t numel, uint16_t *y,
-                         hipStream_t stream) {
+                         const uint8_t *planes, int cols, hipStream_t stream) {
   if (numel == 0) return MOE_STATUS_OK;
   const int64_t blocks = (numel / 4 + 255) / 256;
   hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, ypart,
-                     nsplit, numel, y);
+                     nsplit, numel, y, planes, cols);
   MOE_LAUNCH_CHECK();
   return MOE_STATUS_OK;
 }
@@ -650,7 +676,7 @@ extern "C" int moe_expert_ffn_nf4(const moe_nf4_expert_t *experts, int32_t E, co
   return moe::launch_expert_ffn(experts, E, x_bf16, T, k, H, F, (const int32_t *)counts,
                                 (const int32_t *)offsets, (const int32_t *)perm_tok,
                                 (const int32_t *)active, h_ws_bf16, ypart_f32, nsplit, T, 3,
-                                (hipStream_t)stream, nullptr);
+                                (hipStream_t)stream, nullptr, nullptr);
 }
 
 extern "C" int moe_expert_gateup_nf4(const moe_nf4_expert_t *experts, int32_t E,
@@ -661,7 +687,7 @@ extern "C" int moe_expert_gateup_nf4(const moe_nf4_expert_t *experts, int32_t E,
   return moe::launch_expert_ffn(experts, E, x_bf16, T, k, H, F, (const int32_t *)counts,
                                 (const int32_t *)offsets, (const int32_t *)perm_tok,
                                 (const int32_t *)active, h_ws_bf16, nullptr, 1, T, 1,
-                                (hipStream_t)stream, nullptr);
+                                (hipStream_t)stream, nullptr, nullptr);
 }
 
 extern "C" int moe_expert_down_nf4(const moe_nf4_expert_t *experts, int32_t E, int64_t T,
@@ -672,12 +698,12 @@ extern "C" int moe_expert_down_nf4(const moe_nf4_expert_t *experts, int32_t E, i
   return moe::launch_expert_ffn(experts, E, nullptr, T, k, H, F, (const int32_t *)counts,
                                 (const int32_t *)offsets, (const int32_t *)perm_tok,
                                 (const int32_t *)active, const_cast<void *>(h_ws_bf16),
-                                ypart_f32, nsplit, T, 2, (hipStream_t)stream, nullptr);
+                                ypart_f32, nsplit, T, 2, (hipStream_t)stream, nullptr, nullptr);
 }
 
 extern "C" int moe_combine(const void *ypart_f32, int32_t nsplit, const void *weights_f32,
                            const void *idx_i32, const void *slot_pos, int64_t T, int32_t k,
                            int32_t H, void *out_bf16, void *stream) {
   return moe::launch_combine(ypart_f32, nsplit, weights_f32, idx_i32, slot_pos, T, k, H, out_bf16,
-                             (hipStream_t)stream);
+                             nullptr, 0, (hipStream_t)stream);
 }

@@ -150,6 +150,68 @@ __device__ __forceinline__ uint16_t gm_swiglu_bf16(float g, float u) {
   return f32_to_bf16(sb * ub);
 }
 
+// Down projection in ranges.  Whole items, or K splits of them dealt out one by one, leave CUs
+// idle in the last round, and K splits enough to even that out cost their ypart planes: at
+// 1500 tokens (Mixtral) 8 planes of 49 MB, written here and read by the combine (94 us).  So
+// the items are laid end to end, weighted by what a block of each costs (a partial token
+// tile skips MFMAs but not its weights), and cut into one equal range per workgroup, at
+// 4-block units.  An item cut by range ends has its pieces in successive planes, most items
+// are whole or in two pieces, and the sum reads the planes that an item has.  The cuts depend
+// on the routed counts alone, so results repeat bit for bit.  Down + sum over the
+// planes, 512 tokens: 274 + 25 -> 239 + 14 us; a layer of 512 / 900 / 1500 tokens 612 -> 598,
+// 838 -> 806, 1313 -> 1281 us; hidden 1024 at 300 tokens (32 K-split items before) 108 -> 86;
+// one expert of 128 tokens 203 -> 183 us.  Not for gate/up, whose pieces would have to meet
+// before the SwiGLU: 256 KB of fp32 sums a piece cost a CU about what the round saves.
+constexpr int kMaxRanges = 512;  // workgroups of a launch
+constexpr int kMinPiece = 2;     // units: a shorter piece costs more than it evens out
+
+// Cost of a block of an item with `live` 32-token tiles of MT, in twentieths of a full one.
+template <int MT, bool PIPE>
+__device__ __forceinline__ int gm_cost(int live) {
+  return PIPE || live >= MT ? 20 : 8 + 12 * live / MT;
+}
+
+// s_bound[v]: first unit of workgroup v's range, v <= G.  An item meets at most `planes`
+// ranges: a range holds at least 1 / (planes - 1) of the dearest item's cost.
+template <int MT, bool PIPE>
+__device__ __forceinline__ void gm_bounds(const int (*s_ex)[5], int *s_bound, int n_active, int n_items,
+                                          int wtiles, int U, int G, int planes, int tid, int threads) {
+  // Per expert: cost of one weight tile's token tiles, and of its last (partial) one.
+  auto last_cost = [&](int a) { return gm_cost<MT, PIPE>((s_ex[a][1] - 32 * MT * (s_ex[a][4] - 1) + 31) >> 5); };
+  auto col_cost = [&](int a) { return s_ex[a][4] > 0 ? 20 * (s_ex[a][4] - 1) + last_cost(a) : 0; };
+  uint64_t total = 0;
+  int dear = 1;  // cost of a block of the dearest item
+  for (int a = 0; a < n_active; ++a) {
+    total += (uint64_t)col_cost(a) * (uint64_t)(wtiles * U);
+    dear = max(dear, s_ex[a][4] > 1 ? 20 : s_ex[a][4] == 1 ? last_cost(a) : 0);
+  }
+  const uint64_t most = total * (uint64_t)max(planes - 1, 1) / (uint64_t)(dear * U);
+  const int ways = most < 1 ? 1 : most < (uint64_t)G ? (int)most : G;
+  for (int i = tid; i <= G; i += threads) {
+    int b = n_items * U;
+    if (i < ways) {
+      uint64_t pos = total * (uint64_t)i / (uint64_t)ways;
+      int a = 0;
+      for (; a < n_active - 1; ++a) {
+        const uint64_t c = (uint64_t)col_cost(a) * (uint64_t)(wtiles * U);
+        if (pos < c) break;
+        pos -= c;
+      }
+      const int cu = col_cost(a) * U;
+      if (cu > 0) {
+        const int wt = min((int)(pos / (uint64_t)cu), wtiles - 1);
+        const int r = (int)(pos - (uint64_t)wt * (uint64_t)cu);
+        const int mt = min(r / (20 * U), s_ex[a][4] - 1);
+        int u = (r - mt * 20 * U) / (mt == s_ex[a][4] - 1 ? last_cost(a) : 20);
+        u = min(u, U);
+        u = u < kMinPiece ? 0 : u > U - kMinPiece ? U : u;
+        b = (s_ex[a][3] + wt * s_ex[a][4] + mt) * U + u;
+      }
+    }
+    s_bound[i] = b;
+  }
+}
+
 // The DMA's inline asm names M0, a register the compiler reserves and sets before each of
 // its own uses (this kernel has none besides the asm).
 #pragma clang diagnostic push
@@ -163,7 +225,8 @@ template <bool GATEUP, int W, int MT, int NF, int BD>
 __global__ void __launch_bounds__(W * 64, 1)
 expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint32_t act_bytes,
                    int K, int NROWS, Route rt, int rows_total, int nsplit,
-                   uint16_t *__restrict__ h_out, float *__restrict__ y_out) {
+                   uint16_t *__restrict__ h_out, float *__restrict__ y_out,
+                   uint8_t *__restrict__ planes) {
   constexpr int kGmThreads = W * kWave;
   constexpr int kGmMT = MT;                            // 32-token MFMA tiles per item
   constexpr int kGmM = 32 * MT;                        // tokens per item
@@ -217,6 +280,9 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
   // Three-plane shape: threads whose wave has issued the reads of its current block's plane
   // (counted over the item), in place of a barrier per block.
   __shared__ int s_rdone;
+  // Down with `planes` (see gm_bounds): workgroup v takes the 4-block units [s_bound[v],
+  // s_bound[v + 1]) of the items laid end to end.
+  __shared__ int s_bound[GATEUP ? 1 : kMaxRanges + 1];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -238,7 +304,7 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
       // An absent expert (null pointers) gets no items; the caller routes no token to it.
       cnt = (GATEUP ? tab.e[e].w1_packed : tab.e[e].w2_packed) != nullptr ? rt.counts[e] : 0;
       mtiles = (cnt + kGmM - 1) / kGmM;
-      items = mtiles * nsplit * wtiles;
+      items = mtiles * (planes != nullptr ? 1 : nsplit) * wtiles;
     }
     int incl = items;
 #pragma unroll
@@ -298,7 +364,18 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
   // consecutive items [x G/8, (x + 1) G/8) of every round.
   const int vb = (G & 7) == 0 ? (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3)
                               : (int)blockIdx.x;
-  if (vb >= n_items) return;  // uniform over the workgroup
+  const bool ranges = !GATEUP && planes != nullptr;
+  const int U = NB >> 2;  // units per item
+  int unit = 0, unit_end = 0;
+  if (ranges) {
+    gm_bounds<MT, kPipe>(s_ex, s_bound, n_active, n_items, wtiles, U, G, nsplit, tid, kGmThreads);
+    __syncthreads();
+    unit = __builtin_amdgcn_readfirstlane(s_bound[vb]);
+    unit_end = __builtin_amdgcn_readfirstlane(s_bound[vb + 1]);
+    if (unit >= unit_end) return;  // uniform over the workgroup
+  } else if (vb >= n_items) {
+    return;  // uniform over the workgroup
+  }
 
   auto ex_field = [&](int a, int f) { return __builtin_amdgcn_readfirstlane(s_ex[a][f]); };
   // Item -> (active index, weight tile, split, token tile); wave-uniform.
@@ -309,8 +386,8 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
     const int mtiles = ex_field(a, 4);
     const int q = rem / mtiles;
     mt = rem - q * mtiles;
-    wt = q / nsplit;
-    sp = q - wt * nsplit;
+    wt = planes != nullptr ? q : q / nsplit;
+    sp = planes != nullptr ? 0 : q - wt * nsplit;
   };
 
   // Replica of the lane's table lookups per fragment: with one codebook in the table, lanes
@@ -368,13 +445,38 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
   u32x4 ring[kGmBDepth][kGmNF];
   f32x4 absc[kGmNF], absn[kGmNF];  // absmax of the current and the next group of 4 blocks
 
-  for (int item = vb; item < n_items; item += G) {
+  for (int item = vb; ranges ? unit < unit_end : item < n_items; item += G) {
     int a, wt, sp, mt;
-    decode(item, a, wt, sp, mt);
+    int kb0i, nb;  // blocks kb0i .. kb0i + nb - 1 of the item's K range
+    if (ranges) {
+      item = unit / U;
+      const int lo = item * U, stop = min(unit_end, lo + U);
+      decode(item, a, wt, sp, mt);
+      kb0i = 4 * (unit - lo);
+      nb = 4 * (stop - unit);
+      unit = stop;
+      if (nb < NB) {
+        // One of several pieces of the item: its plane is the number of pieces before it.
+        auto bound = [&](int v) { return __builtin_amdgcn_readfirstlane(s_bound[v]); };
+        for (int v = vb; bound(v) > lo; --v) sp += bound(v) > bound(v - 1) ? 1 : 0;
+      }
+      if (kb0i == 0) {
+        // The item's first piece says how many there are, for the sum over the planes.
+        int n = 1;
+        for (int v = vb + 1; v < G && s_bound[v] < lo + U; ++v) n += s_bound[v + 1] > s_bound[v] ? 1 : 0;
+        const int rows = min(kGmM, ex_field(a, 1) - mt * kGmM);
+        for (int r = tid; r < rows; r += kGmThreads)
+          planes[(size_t)(ex_field(a, 2) + mt * kGmM + r) * wtiles + wt] = (uint8_t)n;
+      }
+    } else {
+      decode(item, a, wt, sp, mt);
+      kb0i = sp * NBp;
+      nb = NBp;
+    }
     if (tbl_a < 0 || (per_item_table && a != tbl_a)) build_table(a);
     const int cnt = ex_field(a, 1), off = ex_field(a, 2);
     const uint32_t row0 = (uint32_t)(wt * kRowsItem + wave * kRowsWave);
-    const uint32_t kb0 = (uint32_t)(sp * NBp);
+    const uint32_t kb0 = (uint32_t)kb0i;
     auto uptr = [&](int f) {
       const uint64_t v = (uint64_t)(uintptr_t)s_ptr[a][f];
       const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
@@ -409,12 +511,12 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
     // Weights of block b and absmax of blocks b4..b4+3 (past the split's end: its last
     // block / group again, unused).
     auto load_b = [&](int slot, int b) {
-      const uint32_t bo = w_lane + (uint32_t)(b < NBp ? b : NBp - 1) * 32u;
+      const uint32_t bo = w_lane + (uint32_t)(b < nb ? b : nb - 1) * 32u;
 #pragma unroll
       for (int f = 0; f < kGmNF; ++f) ring[slot][f] = *reinterpret_cast<const GM_GLOBAL u32x4 *>(wb[f] + bo);
     };
     auto load_s = [&](f32x4 (&dst)[kGmNF], int b4) {
-      const uint32_t so = s_lane + (uint32_t)(b4 < NBp ? b4 : NBp - 4);
+      const uint32_t so = s_lane + (uint32_t)(b4 < nb ? b4 : nb - 4);
 #pragma unroll
       for (int f = 0; f < kGmNF; ++f) dst[f] = *reinterpret_cast<const GM_GLOBAL f32x4 *>(ab[f] + so);
     };
@@ -423,7 +525,7 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
     // LDS reads wait for them (it cannot tell the planes apart); the explicit vmcnt waits
     // before the barriers count them.  M0 holds the wave's 1 KB destination.
     auto dma = [&](uint32_t plane, int b) {
-      const uint32_t adv = (uint32_t)(b < NBp ? b : NBp - 1) * 128u;
+      const uint32_t adv = (uint32_t)(b < nb ? b : nb - 1) * 128u;
 #pragma unroll
       for (int j = 0; j < kGmFill; ++j) {
         const uint32_t dst = plane + (uint32_t)(8 * W * j + 8 * wave) * 128u;
@@ -585,10 +687,10 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
     // batch spill a few rows past 128).
     live = min(kGmMT, (cnt - mt * kGmM + 31) >> 5);
     int pb = 0;  // plane of block b: b % kPlanes
-    for (int b0 = 0; b0 < NBp; b0 += kGmBDepth) {
+    for (int b0 = 0; b0 < nb; b0 += kGmBDepth) {
 #pragma unroll
       for (int d = 0; d < kGmBDepth; ++d) {
-        if (BD == 4 || b0 + d < NBp) {  // a split (4 k blocks) may end inside a BD-block step
+        if (BD == 4 || b0 + d < nb) {  // a split (4 k blocks) may end inside a BD-block step
           // Plane (b + kLA) % kPlanes = (b - 1) % kPlanes was last read in block b - 1,
           // before the barrier.
           const int pd = pb == 0 ? kPlanes - 1 : pb - 1;
@@ -702,22 +804,55 @@ int expert_gemm_splits(int64_t rows, int64_t active, int32_t H, int32_t F) {
 template <int W, int MT, int NF, int BD>
 static int launch_gemm_shape(const ExpertTable &tab, const void *x, int64_t T, int64_t rows_total,
                              int32_t H, int32_t F, const Route &rt, void *h_ws, void *ypart,
-                             int32_t nsplit, int phases, hipStream_t stream) {
+                             int32_t nsplit, int phases, uint8_t *planes, hipStream_t stream) {
   const dim3 grid((unsigned)device_cu_count()), blk(W * kWave);
   if (phases & 1) {
     hipLaunchKernelGGL((expert_gemm_kernel<true, W, MT, NF, BD>), grid, blk, 0, stream, tab,
                        (const uint16_t *)x, (uint32_t)(T * H * 2), H, F, rt, (int)rows_total, 1,
-                       (uint16_t *)h_ws, (float *)nullptr);
+                       (uint16_t *)h_ws, (float *)nullptr, (uint8_t *)nullptr);
     MOE_LAUNCH_CHECK();
   }
   if (phases & 2) {
     hipLaunchKernelGGL((expert_gemm_kernel<false, W, MT, NF, BD>), grid, blk, 0, stream, tab,
                        (const uint16_t *)h_ws, (uint32_t)(rows_total * F * 2), F, H, rt,
-                       (int)rows_total, nsplit, (uint16_t *)nullptr, (float *)ypart);
+                       (int)rows_total, nsplit, (uint16_t *)nullptr, (float *)ypart, planes);
     MOE_LAUNCH_CHECK();
   }
   return MOE_STATUS_OK;
 }
+
+// Planes for a down projection in ranges: pieces that an item of the expected routing (rows
+// spread evenly) can have with one range per CU, and one more for uneven routing.
+int expert_gemm_planes(int64_t rows, int64_t active, int32_t H, int32_t F) {
+  const GemmShape g = gemm_shape(rows, active);
+  const int64_t per = active > 0 ? (rows + active - 1) / active : 0;
+  const int64_t items = active * ((per + g.tokens() - 1) / g.tokens()) * (H / g.down_rows());
+  const int64_t n = items > 0 ? (device_cu_count() + items - 1) / items + 2 : 1;
+  return (int)(n < 2 ? 2 : n > 16 ? 16 : n);
+}
+// Whether a layer's down projection runs in ranges.  Not
+//  * with 256-token items of four or more experts: 2 rounds of items or more, whose launch is
+//    bound by the clock that the chip's power allows, and items dealt out one by one share
+//    their operands in L2 (T = 4096: 2795 us a layer, 2930 in ranges; one expert of 2048
+//    tokens: 752 us in whole K splits, 667 in ranges);
+//  * where K splits fill every round for any routing near the average, through cheap planes
+//    (16 experts, top-4, hidden 2048, 300 tokens: 235 us, 250 in ranges, which start and end
+//    inside items).
+bool expert_gemm_ranges_ok(int64_t rows, int64_t active, int32_t H, int32_t F) {
+  if (device_cu_count() > kMaxRanges || active < 1) return false;
+  const GemmShape g = gemm_shape(rows, active);
+  if (g.mt == 8 && active >= 4) return false;
+  const int64_t cus = device_cu_count();
+  const int64_t per = (rows + active - 1) / active, m = g.tokens();
+  int64_t sd = 1;  // standard deviation of an expert's rows
+  while (active > 1 && (sd + 1) * (sd + 1) <= per) ++sd;
+  const bool steady = active == 1 || (per - 2 * sd > 0 && (per - 2 * sd + m - 1) / m == (per + 2 * sd + m - 1) / m);
+  const int64_t s = gemm_splits_for(g, rows, active, H, F);
+  const int64_t pieces = active * ((per + m - 1) / m) * (H / g.down_rows()) * s;
+  const int64_t rounds = (pieces + cus - 1) / cus;
+  return !(steady && 10 * pieces >= 9 * rounds * cus && s * rows * H * 4 <= (int64_t)40 << 20);
+}
+int expert_gemm_down_cols(int64_t rows, int64_t active) { return (int)gemm_shape(rows, active).down_rows(); }
 
 static int check_gemm_args(int64_t T, int64_t rows_total, int32_t H, int32_t F, int32_t nsplit) {
   MOE_REQUIRE(expert_gemm_supported(H, F), "shape not supported by the batched expert GEMM");
@@ -728,15 +863,15 @@ static int check_gemm_args(int64_t T, int64_t rows_total, int32_t H, int32_t F, 
 
 int launch_expert_gemm(const void *tab_v, const void *x, int64_t T, int64_t rows_total,
                        int64_t active_max, int32_t H, int32_t F, const void *route_v, void *h_ws,
-                       void *ypart, int32_t nsplit, int phases, hipStream_t stream) {
-  const int rc = check_gemm_args(T, rows_total, H, F, nsplit);
+                       void *ypart, int32_t nsplit, int phases, uint8_t *planes, hipStream_t stream) {
+  const int rc = check_gemm_args(T, rows_total, H, F, planes ? 1 : nsplit);
   if (rc != MOE_STATUS_OK) return rc;
   const ExpertTable &tab = *static_cast<const ExpertTable *>(tab_v);
   const Route &rt = *static_cast<const Route *>(route_v);
   const GemmShape g = gemm_shape(rows_total, active_max);
   if (g.mt == 8)
-    return launch_gemm_shape<4, 8, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, stream);
-  return launch_gemm_shape<8, 4, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, stream);
+    return launch_gemm_shape<4, 8, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, planes, stream);
+  return launch_gemm_shape<8, 4, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, planes, stream);
 }
 
 }  // namespace moe

@@ -600,3 +600,42 @@ def test_mid_down_needs_a_workgroup_per_pair(cuda_device):
     assert ops.choose_nsplit(64, 2, 8, 2048, 14336) == 7
     if (32 + 64 * 2 // 16) * 7 > cus:
         assert ops.choose_nsplit(64, 2, 32, 2048, 14336) != 7
+
+
+# ------------------------------------------------------------------------------ batched GEMM
+@pytest.mark.parametrize("T,k,E,H,F,skew", [
+    (128, 1, 1, 512, 768, 0.0),        # one 128-row item per weight tile, 3 units of K
+    (129, 1, 1, 1024, 3584, 0.0),      # a second item of one row
+    (160, 2, 4, 512, 256, 0.0),        # one unit of K: nothing to cut
+    (300, 2, 8, 1024, 3584, 0.0),      # fewer items than CUs
+    (333, 2, 8, 1024, 2048, 3.0),      # experts with few rows and none
+    (900, 4, 16, 512, 1024, 1.0),
+    (641, 1, 1, 1024, 1792, 0.0),      # 256-row items, the last one half empty (129 rows)
+    (640, 1, 1, 1024, 1792, 0.0),      # its last one of 128 rows: half of the token tiles
+    (1600, 2, 3, 512, 1024, 0.5),
+])
+def test_down_in_ranges(cuda_device, T, k, E, H, F, skew):
+    """A layer's down projection in ranges (items cut by equal shares of the work, their pieces
+    in as many ypart planes as each has) against the same layer through the separate calls,
+    with whole items in one plane: fp32 sums in another order, so single bf16 roundings of
+    the output differ (2^-9 of a value, on a small share of them)."""
+    from moeinfra_amd import ops
+    from moeinfra_amd._lib import MoeNf4Expert
+
+    g = torch.Generator(device=cuda_device).manual_seed(T + F)
+    keep = [{n: ops.nf4_quantize((torch.randn(s, generator=g, device=cuda_device) * 0.02).to(torch.bfloat16))
+             for n, s in (("w1", (F, H)), ("w3", (F, H)), ("w2", (H, F)))} for _ in range(E)]
+    table = ops.expert_table([MoeNf4Expert(*(t.data_ptr() for n in ("w1", "w3", "w2") for t in st[n]))
+                              for st in keep])
+    gate = (torch.randn((E, H), generator=g, device=cuda_device) * 0.02).to(torch.bfloat16)
+    x = torch.randn((T, H), generator=g, device=cuda_device).to(torch.bfloat16)
+    bias = -skew * torch.arange(E, dtype=torch.float32, device=cuda_device)
+    out, _, w, idx = ops.layer_forward(table, E, gate, x, k, F, bias=bias)
+    again, _, _, _ = ops.layer_forward(table, E, gate, x, k, F, bias=bias)
+    assert torch.equal(out, again)
+    idx32 = idx.to(torch.int32)
+    route = ops.permute(idx32, E)
+    _, ypart = ops.expert_ffn(table, E, x, k, H, F, route, nsplit=1)
+    want = ops.combine(ypart, w, idx32, route["slot_pos"])
+    assert orc.rel_l2(out.float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-3
+    assert (out != want).float().mean() < 0.1
