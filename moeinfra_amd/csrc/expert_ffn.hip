@@ -463,6 +463,7 @@ int launch_skinny(const void *tab, const void *x, int64_t T, int64_t rows_total,
 bool midbatch_supported(int32_t H, int32_t F, int32_t nsplit);
 bool midbatch_rows_ok(int64_t T, int64_t rows_total, int32_t H, int32_t F);
 int midbatch_splits(int64_t active_max, int32_t H, int32_t F);
+bool midbatch_gateup_fills(int64_t active_max, int32_t F);
 int launch_midbatch(const void *tab, const void *x, int64_t T, int64_t rows_total, int32_t H,
                     int32_t F, const void *route, void *h_ws, void *ypart, int32_t nsplit,
                     int phases, hipStream_t stream);
@@ -530,6 +531,22 @@ int launch_mid_layer_gateup(const moe_nf4_expert_t *experts, int32_t E, const vo
   return launch_mid_gateup(&tab, x, T, k, H, F, E, nullptr, h_ws, stream, route_out);
 }
 
+// Gate/up of the batched GEMM on the 32-row x 32-token items of the K-split form instead: its
+// 256-row items fill one round of the CUs at most, and the small ones, which stream the
+// weights once per 32 rows of an expert, take up to seven.  One expert of hidden 1024, F 3584
+// at 64 / 256 / 400 / 1000 rows: 60 / 75 / 75 / 80 us a call on the GEMM, 43 / 60 / 70 / 107
+// so; hidden 3072, F 8192 at 64 / 200 / 400: 117 / 147 / 154 and 71 / 131 / 197; hidden 4096,
+// F 14336 at 100 / 150: 177 / 179 and 155 / 193; a layer of 8 experts, hidden 1024, at 130 /
+// 200 tokens: 80 / 80 and 76 / 82.  (Half a chunk is added for uneven rows.)
+bool small_gateup(int64_t T, int64_t rows, int64_t active, int32_t H, int32_t F) {
+  const int64_t cus = device_cu_count();
+  const int64_t per = active > 0 ? (rows + active - 1) / active : 0;
+  const int64_t chunks = (per + (active > 1 ? 16 : 0) + 31) / 32;
+  return skinny_supported(H, F) && rows <= 2048 && T * (int64_t)H * 2 < ((int64_t)1 << 31) &&
+         rows * (int64_t)F * 2 < ((int64_t)1 << 31) && active * ((per + 127) / 128) * (F / 256) <= cus &&
+         active * chunks * (F / 32) <= 7 * cus;
+}
+
 // phases: bit 0 = gate/up (x -> h), bit 1 = down (h -> ypart).  Up to 4 tokens per expert
 // use the 4x4x4 MFMA GEMV (expert_gemv4.hip); more use the 16x16x32 tiles below.
 int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x, int64_t T,
@@ -587,15 +604,27 @@ int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x,
   // 128 tokens (the per-tile kernels below re-stream it every 16 or 32 tokens).
   if (fused == nullptr && rows_total >= kGemmMinRowsPerExpert * active_max &&
       expert_gemm_supported(H, F) && (planes != nullptr || expert_gemm_splits_ok(F, nsplit)) &&
-      expert_gemm_rows_ok(T, rows_total, H, F))
+      expert_gemm_rows_ok(T, rows_total, H, F)) {
+    if ((phases & 1) && small_gateup(T, rows_total, active_max, H, F)) {
+      const int rc = launch_skinny(&tab, x, T, rows_total, H, F, &rt, h_ws, ypart, 1, stream);
+      if (rc != MOE_STATUS_OK || !(phases & 2)) return rc;
+      phases &= ~1;
+    }
     return launch_expert_gemm(&tab, x, T, rows_total, active_max, H, F, &rt, h_ws, ypart, nsplit,
                               phases, planes, stream);
+  }
   // Fewer: the mid-batch kernels stream each weight tile once per 32 tokens of its expert
   // (32x32x16 MFMA, 16-byte weight loads): the streamed form (whole-K waves, activations
   // through LDS, `nsplit` K splits of the down projection) where the shape allows, else the
   // K-split form with activations from L2.
-  if (fused == nullptr && midbatch_supported(H, F, nsplit) && midbatch_rows_ok(T, rows_total, H, F))
+  if (fused == nullptr && midbatch_supported(H, F, nsplit) && midbatch_rows_ok(T, rows_total, H, F)) {
+    if ((phases & 1) && rows_total <= 2048 && !midbatch_gateup_fills(active_max, F)) {
+      const int rc = launch_skinny(&tab, x, T, rows_total, H, F, &rt, h_ws, ypart, 1, stream);
+      if (rc != MOE_STATUS_OK || !(phases & 2)) return rc;
+      phases &= ~1;
+    }
     return launch_midbatch(&tab, x, T, rows_total, H, F, &rt, h_ws, ypart, nsplit, phases, stream);
+  }
   if (nsplit == 1 && fused == nullptr && skinny_supported(H, F) && rows_total <= 2048 &&
       T * (int64_t)H * 2 < ((int64_t)1 << 31) && rows_total * (int64_t)F * 2 < ((int64_t)1 << 31))
     return launch_skinny(&tab, x, T, rows_total, H, F, &rt, h_ws, ypart, phases, stream);

@@ -639,3 +639,26 @@ def test_down_in_ranges(cuda_device, T, k, E, H, F, skew):
     want = ops.combine(ypart, w, idx32, route["slot_pos"])
     assert orc.rel_l2(out.float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-3
     assert (out != want).float().mean() < 0.1
+
+
+@pytest.mark.parametrize("T,k,E,H,F", [
+    (13, 2, 8, 1024, 3584),     # seven K splits of the down projection, gate/up K-split
+    (9, 2, 4, 512, 1536),       # three
+    (20, 1, 1, 1024, 3584),     # one expert: both
+    (31, 1, 1, 512, 4096),
+    (33, 1, 1, 1024, 3584),     # batched GEMM, gate/up on small items
+    (129, 1, 1, 512, 1024),
+    (140, 2, 8, 1024, 2048),
+])
+def test_few_items_layer(cuda_device, T, k, E, H, F):
+    """Layers whose weight tiles are few for the CUs (gate/up on the K-split form, the down
+    projection in as many K splits as its shape allows) against the CPU oracle."""
+    gate, experts, x = build_layer(H, F, E, T, seed=T + F)
+    want, (lg, _, _) = oracle_layer(gate, experts, x, k)
+    from moeinfra_amd import ops
+
+    table = ops.expert_table([e.to(cuda_device).c_struct() for e in experts])
+    out, _, _, _ = ops.layer_forward(table, E, gate.to(cuda_device), x.to(cuda_device), k, F)
+    ok = ~near_tie_rows(lg, k=k, slack=logit_slack(bits(x), bits(gate)))
+    got = orc.bf16_to_f32(bits(out))[ok]
+    assert orc.rel_l2(got, orc.bf16_to_f32(want)[ok]) <= 1e-2
