@@ -476,6 +476,16 @@ int launch_mid_gateup(const void *tab, const void *x, int64_t T, int32_t k, int3
                       int32_t E, const void *route, void *h_ws, hipStream_t s,
                       const void *route_out);
 
+// Up to 4 tokens per expert run the 4x4x4 MFMA GEMV.  A lone expert does not where the mid-size
+// kernels or the K-split items take its shape: the GEMV's work grows with the tokens and one
+// expert's rows do not fill the chip with it (H = 4096, F = 14336, 1 / 2 / 4 tokens: 48 / 52 /
+// 64 us a call, 43 / 44 / 44 with the mid-size kernels; H = 3072: 36 / 39 / 47 and 36 / 36 /
+// 37; layers of 16 experts are 4 % faster with it).
+bool gemv4_chosen(int64_t max_tokens, int32_t E, int32_t H, int32_t F) {
+  return gemv4_supported(max_tokens, H, F) &&
+         !(E == 1 && (mid_gateup_supported(max_tokens, 1, 1, H, F) || midbatch_supported(H, F, 1)));
+}
+
 // ypart planes a layer's down projection writes (the combine adds them): the streamed
 // mid-batch kernels split K of the down projection over workgroups when few experts would
 // leave CUs idle; every other path writes one plane.  Follows the path choice of
@@ -483,7 +493,7 @@ int launch_mid_gateup(const void *tab, const void *x, int64_t T, int32_t k, int3
 int choose_nsplit(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F) {
   const int64_t rows = T * k;
   const int64_t active_max = rows < E ? rows : E;
-  if (T <= 0 || gemv4_supported(T, H, F)) return 1;
+  if (T <= 0 || gemv4_chosen(T, E, H, F)) return 1;
   if (mid_down_supported(T, k, E, H, F)) return mid_down_parts(F);
   if (rows >= kGemmMinRowsPerExpert * active_max && expert_gemm_supported(H, F) &&
       expert_gemm_rows_ok(T, rows, H, F))
@@ -497,7 +507,7 @@ int choose_nsplit(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F) {
 int layer_range_planes(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, int *cols) {
   const int64_t rows = T * k;
   const int64_t active_max = rows < E ? rows : E;
-  if (T <= 0 || gemv4_supported(T, H, F) || mid_down_supported(T, k, E, H, F) ||
+  if (T <= 0 || gemv4_chosen(T, E, H, F) || mid_down_supported(T, k, E, H, F) ||
       rows < kGemmMinRowsPerExpert * active_max || !expert_gemm_supported(H, F) ||
       !expert_gemm_rows_ok(T, rows, H, F) || !expert_gemm_ranges_ok(rows, active_max, H, F))
     return 0;
@@ -584,7 +594,7 @@ int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x,
   const int64_t wg_cap = (int64_t)device_cu_count() * 2;
   const int mt = token_tiles_for(max_tokens_per_expert);
 
-  if (nsplit == 1 && gemv4_supported(max_tokens_per_expert, H, F))
+  if (nsplit == 1 && gemv4_chosen(max_tokens_per_expert, E, H, F))
     return launch_gemv4(&tab, x, H, F, &rt, h_ws, ypart, phases, active_max, rows_total, fused,
                         stream);
   // Mid-size batches (up to 64 tokens): gate/up on 16-row weight tiles of "virtual experts"

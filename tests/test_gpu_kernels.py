@@ -662,3 +662,16 @@ def test_few_items_layer(cuda_device, T, k, E, H, F):
     ok = ~near_tie_rows(lg, k=k, slack=logit_slack(bits(x), bits(gate)))
     got = orc.bf16_to_f32(bits(out))[ok]
     assert orc.rel_l2(got, orc.bf16_to_f32(want)[ok]) <= 1e-2
+
+
+@pytest.mark.parametrize("T", [1, 2, 4, 5])
+@pytest.mark.parametrize("H,F", [(2048, 2048), (1024, 3584), (512, 1024), (256, 768)])
+def test_lone_expert_few_tokens(cuda_device, T, H, F):
+    """One expert on 1 to 5 rows: the mid-size kernels, the K-split items, and the GEMV where
+    neither takes the shape, against the CPU oracle."""
+    from moeinfra_amd import ops
+
+    _, (expert,), x = build_layer(H, F, 1, T, seed=T + H)
+    want = orc.bf16_to_f32(orc.swiglu(bits(x), *expert.dequant_np()))
+    got = ops.expert_swiglu(expert.to(cuda_device).c_struct(), x.to(cuda_device), H, F)
+    assert orc.rel_l2(orc.bf16_to_f32(bits(got)), want) <= 1e-2
