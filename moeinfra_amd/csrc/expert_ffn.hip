@@ -326,6 +326,9 @@ down_kernel(const ExpertTable tab, int H, int F, Route rt, const uint16_t *__res
 constexpr int kCombineThreads = 64;
 constexpr int kCombineCols = kCombineThreads * 4;
 
+// RANGES: the down projection ran in ranges, and a row's item has planes[...] planes instead of
+// nsplit (a form of its own: the extra load ahead of the sums costs the others 1 us).
+template <bool RANGES>
 __global__ void __launch_bounds__(kCombineThreads)
 combine_kernel(const float *__restrict__ ypart, int nsplit, int64_t rows_total,
                const float *__restrict__ wts, const int32_t *__restrict__ idx,
@@ -358,8 +361,7 @@ combine_kernel(const float *__restrict__ ypart, int nsplit, int64_t rows_total,
     if (pos < 0 || pos >= rows_total) continue;
     const float w = wts[t * k + j];
     float4 y = *reinterpret_cast<const float4 *>(ypart + (size_t)pos * H + c);
-    // Planes of this row's item: all, or as many as it has pieces (cols output columns each).
-    const int np = planes != nullptr ? planes[(size_t)pos * (H / cols) + c / cols] : nsplit;
+    const int np = RANGES ? planes[(size_t)pos * (H / cols) + c / cols] : nsplit;
 #pragma unroll 4
     for (int s = 1; s < np; ++s) {
       const float4 v = *reinterpret_cast<const float4 *>(ypart + s * split_stride + (size_t)pos * H + c);
@@ -392,6 +394,7 @@ __global__ void identity_route_kernel(int64_t T, int32_t *counts, int32_t *offse
   }
 }
 
+template <bool RANGES>
 __global__ void reduce_splits_kernel(const float *__restrict__ ypart, int nsplit, int64_t numel,
                                      uint16_t *__restrict__ y, const uint8_t *__restrict__ planes,
                                      int cols) {
@@ -399,8 +402,7 @@ __global__ void reduce_splits_kernel(const float *__restrict__ ypart, int nsplit
   if (i >= numel) return;
   float4 acc = *reinterpret_cast<const float4 *>(ypart + i);
   // Row i / H's items follow each other in `planes`, cols columns each (H a multiple).
-  const int np = planes != nullptr ? planes[i / cols] : nsplit;
-#pragma unroll 4
+  const int np = RANGES ? planes[i / cols] : nsplit;
   for (int s = 1; s < np; ++s) {
     const float4 v = *reinterpret_cast<const float4 *>(ypart + (size_t)s * numel + i);
     acc.x += v.x;
@@ -679,7 +681,8 @@ int launch_combine(const void *ypart, int32_t nsplit, const void *weights, const
   MOE_REQUIRE(((uintptr_t)ypart % 16) == 0 && ((uintptr_t)out % 8) == 0,
               "ypart must be 16-byte and out 8-byte aligned");
   const unsigned cgrid = (unsigned)((H + kCombineCols - 1) / kCombineCols);
-  hipLaunchKernelGGL(combine_kernel, dim3((unsigned)T, cgrid), dim3(kCombineThreads), 0, stream,
+  auto kern = planes != nullptr ? combine_kernel<true> : combine_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)T, cgrid), dim3(kCombineThreads), 0, stream,
                      (const float *)ypart, nsplit, T * k, (const float *)weights,
                      (const int32_t *)idx_i32, (const int32_t *)slot_pos, k, H, (uint16_t *)out,
                      planes, cols);
@@ -700,7 +703,8 @@ int launch_reduce_splits(const float *ypart, int nsplit, int64_t numel, uint16_t
                          const uint8_t *planes, int cols, hipStream_t stream) {
   if (numel == 0) return MOE_STATUS_OK;
   const int64_t blocks = (numel / 4 + 255) / 256;
-  hipLaunchKernelGGL(reduce_splits_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, ypart,
+  auto kern = planes != nullptr ? reduce_splits_kernel<true> : reduce_splits_kernel<false>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(256), 0, stream, ypart,
                      nsplit, numel, y, planes, cols);
   MOE_LAUNCH_CHECK();
   return MOE_STATUS_OK;
