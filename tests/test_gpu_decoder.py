@@ -589,3 +589,41 @@ def test_engine_rejects_bad_requests(cuda_device):
         eng.generate(ForwardRequest(torch.zeros((1, 20), dtype=torch.long)))
     with pytest.raises(ValueError):
         eng.generate(ForwardRequest(torch.zeros((1, 4), dtype=torch.long), max_new_tokens=-1))
+
+
+def test_long_context_step_replays(cuda_device):
+    """Decode steps that cross the length from which workgroups share a row's keys (384): a
+    captured step, replayed with the program's own eager prefill between the replays, gives
+    the bits of eager steps, and forward() of one token those of decode_step()."""
+    from moeinfra_amd.engine.decoder import MixtralShape, NativeDecoder, synthesize
+
+    shape = MixtralShape(hidden=512, ffn=512, layers=2, n_heads=8, n_kv_heads=2, head_dim=64, vocab=640)
+    w = synthesize(shape, seed=11, device=cuda_device)
+    ids = torch.randint(0, shape.vocab, (381,), generator=torch.Generator().manual_seed(4)).to(cuda_device)
+    a, b, c, other = (NativeDecoder(w, 640, cuda_device) for _ in range(4))
+    for d in (a, b, c):
+        d.forward(ids)
+    np.testing.assert_array_equal(bits(a.k_cache), bits(b.k_cache))
+    toks = {d: ids[:1].clone() for d in (a, b, c)}
+    a_pos, side = b.pos.clone(), torch.cuda.Stream(cuda_device)
+    kv = b.k_cache.clone(), b.v_cache.clone()
+    side.wait_stream(torch.cuda.current_stream(cuda_device))
+    with torch.cuda.stream(side):
+        b.decode_step(toks[b])
+    torch.cuda.current_stream(cuda_device).wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        lg = b.decode_step(toks[b])
+    b.pos.copy_(a_pos), b.k_cache.copy_(kv[0]), b.v_cache.copy_(kv[1]), toks[b].copy_(ids[:1])
+    for step in range(7):                       # positions 381 .. 387
+        want = a.decode_step(toks[a]).clone()
+        graph.replay()
+        other.reset()
+        other.forward(ids[:40 + step])          # eager work of another decoder
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(bits(lg), bits(want))
+        got = c.forward(toks[c])
+        np.testing.assert_array_equal(bits(got), bits(want))
+        toks[c].copy_(toks[a])
+        assert torch.equal(toks[a], toks[b])
+    assert not b._attn_ws[:4096].any()

@@ -653,7 +653,9 @@ def test_down_in_ranges(cuda_device, T, k, E, H, F, skew):
 def test_few_items_layer(cuda_device, T, k, E, H, F):
     """Layers whose weight tiles are few for the CUs (gate/up on the K-split form, the down
     projection in as many K splits as its shape allows) against the CPU oracle."""
-    gate, experts, x = build_layer(H, F, E, T, seed=T + F)
+    # The last expert holds a codebook of its own.
+    codes = {E - 1: np.linspace(-1.0, 1.0, 16, dtype=np.float32)}
+    gate, experts, x = build_layer(H, F, E, T, seed=T + F, codes=codes)
     want, (lg, _, _) = oracle_layer(gate, experts, x, k)
     from moeinfra_amd import ops
 
