@@ -280,9 +280,11 @@ few_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict_
     for (int w = 1; w < kAttnThreads / kWave; ++w) mx = fmaxf(mx, s_red[w]);
     __syncthreads();
   }
+  // A split whose scores are all -inf: any finite reference (its probabilities are zero).
+  const float mref = !whole && mx == -INFINITY ? 0.0f : mx;
   float sum = 0.0f;
   for (int j = threadIdx.x; j < n; j += kAttnThreads) {
-    const float e = expf(s_p[j] - mx);
+    const float e = expf(s_p[j] - mref);
     s_p[j] = e;
     sum += e;
   }

@@ -207,6 +207,42 @@ def test_attention_nonfinite_values(cuda_device, T, p0, hd):
         assert rel_l2(got.masked_fill(hit, 0.0), want.masked_fill(hit, 0.0)) < 4e-3
 
 
+@pytest.mark.parametrize("T", [1, 8, 40])
+@pytest.mark.parametrize("lost", ["one pass", "one NaN", "all"])
+def test_attention_scores_of_minus_infinity(cuda_device, T, lost):
+    """Keys whose scores overflow to -inf have probability zero, also where they are all that a
+    workgroup sharing the row's keys has (128 keys a pass at head dim 128); a NaN among them,
+    or no finite score at all, gives NaN as in the module's softmax."""
+    from moeinfra_amd import _lib
+
+    nq, nkv, hd, p0, max_seq = 8, 2, 128, 1000, 2048
+    S = p0 + T
+    q, k, v = _bf16((T, nq, hd), 25).abs() + 0.125, _bf16((nkv, S, hd), 26), _bf16((nkv, S, hd), 27)
+    if lost == "all":
+        k[:] = -3e38
+    else:
+        k[:, 128:256] = -3e38
+    if lost == "one NaN":
+        k[1, 200, 5] = float("nan")
+    kc = torch.zeros((nkv, max_seq, hd), dtype=torch.bfloat16)
+    vc = kc.clone()
+    kc[:, :S], vc[:, :S] = k, v
+    n = _lib.lib().moe_attention_workspace_bytes(T, nq, nkv, hd, max_seq)
+    ws = torch.zeros((n,), dtype=torch.uint8, device=cuda_device)
+    want = _attend_ref(q, k, v, p0).reshape(T, nq, hd)
+    nan = torch.zeros((T, nq, hd), dtype=torch.bool)
+    if lost != "one pass":
+        nan[:, 0 if lost == "all" else nq // 2:] = True
+    assert torch.equal(torch.isnan(want), nan)
+    for w in (None, ws):
+        got = _attend(q.to(cuda_device), kc.to(cuda_device), vc.to(cuda_device), p0, w)
+        got = got.cpu().float().reshape(T, nq, hd)
+        assert torch.equal(torch.isnan(got), nan)
+        if lost != "all":
+            # As test_attention: bf16 rounding of the probabilities and of the output.
+            assert rel_l2(got.masked_fill(nan, 0.0), want.masked_fill(nan, 0.0)) < 4e-3
+
+
 @pytest.mark.parametrize("T,N,K", [(1, 6144, 4096), (1, 4096, 4096), (1, 1000, 512), (4, 515, 1024)])
 def test_gemv(cuda_device, T, N, K):
     from moeinfra_amd import _lib
