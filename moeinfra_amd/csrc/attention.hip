@@ -434,7 +434,7 @@ __device__ __noinline__ void fa_rows_scalar(const uint16_t *q, const char *kbase
       const float mn = fmaxf(m, mx[0]);
       const float mref = mn == -INFINITY ? 0.0f : mn;
       const float alpha = __builtin_amdgcn_exp2f((m - mref) * kLog2e);
-      const float p = __builtin_amdgcn_exp2f(fmaf(x, kLog2e, -mref * kLog2e));
+      const float p = __builtin_amdgcn_exp2f((x - mref) * kLog2e);
       m = mn;
       l = l * alpha + wave_sum(p);
       for (int e = 0; e < HD / kWave; ++e) o[e] *= alpha;
@@ -655,15 +655,15 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
         for (int v = 0; v < 16; ++v) acc[dt][v] *= alpha;
       m = mn;
     }
-    const float nref = -mref * kLog2e;
     u32x4 pf[4];
 #pragma unroll
     for (int s = 0; s < 4; ++s)
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int v = 8 * (s & 1) + 2 * j;
-        const float e0 = __builtin_amdgcn_exp2f(fmaf(sc[s >> 1][v], kLog2e, nref));
-        const float e1 = __builtin_amdgcn_exp2f(fmaf(sc[s >> 1][v + 1], kLog2e, nref));
+        // (The difference first: mref * kLog2e alone overflows from 2.36e38.)
+        const float e0 = __builtin_amdgcn_exp2f((sc[s >> 1][v] - mref) * kLog2e);
+        const float e1 = __builtin_amdgcn_exp2f((sc[s >> 1][v + 1] - mref) * kLog2e);
         l += e0 + e1;
         pf[s][j] = pack_bf16x2(e0, e1);
       }

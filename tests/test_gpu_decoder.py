@@ -116,7 +116,7 @@ def test_attention(cuda_device, T, p0, max_seq, hd):
     assert rel_l2(out.cpu(), want) < 4e-3
 
 
-def _attend(q, kc, vc, p0, ws):
+def _attend(q, kc, vc, p0, ws, scaling=None):
     """moe_attention_ws_bf16 (moe_attention_bf16 with ws None) of q [T, nq, hd] on the GPU."""
     from moeinfra_amd import _lib
 
@@ -124,7 +124,7 @@ def _attend(q, kc, vc, p0, ws):
     out = torch.empty((T, nq * hd), dtype=torch.bfloat16, device=q.device)
     pos = torch.tensor([p0], dtype=torch.int32, device=q.device)
     args = (q.data_ptr(), kc.data_ptr(), vc.data_ptr(), T, nq, nkv, hd, pos.data_ptr(), max_seq,
-            hd ** -0.5, out.data_ptr())
+            hd ** -0.5 if scaling is None else scaling, out.data_ptr())
     st = torch.cuda.current_stream().cuda_stream
     if ws is None:
         _lib.check(_lib.lib().moe_attention_bf16(*args, st), "attention")
@@ -133,7 +133,7 @@ def _attend(q, kc, vc, p0, ws):
     return out
 
 
-def _attend_ref(q, k, v, p0):
+def _attend_ref(q, k, v, p0, scaling=None):
     """Eager attention in fp32 with the bf16 roundings of the bf16 module, one query at a time
     over the keys that it sees."""
     T, nq, hd = q.shape
@@ -143,7 +143,7 @@ def _attend_ref(q, k, v, p0):
         K = k[:, :p0 + t + 1].float().repeat_interleave(grp, dim=0)
         V = v[:, :p0 + t + 1].float().repeat_interleave(grp, dim=0)
         sc = torch.einsum("hd,hkd->hk", q[t].float(), K).to(torch.bfloat16)
-        sc = (sc.float() * hd ** -0.5).to(torch.bfloat16).float()
+        sc = (sc.float() * (hd ** -0.5 if scaling is None else scaling)).to(torch.bfloat16).float()
         p = torch.softmax(sc, dim=-1).to(torch.bfloat16).float()
         out[t] = torch.einsum("hk,hkd->hd", p, V)
     return out.reshape(T, -1)
@@ -241,6 +241,43 @@ def test_attention_scores_of_minus_infinity(cuda_device, T, lost):
         if lost != "all":
             # As test_attention: bf16 rounding of the probabilities and of the output.
             assert rel_l2(got.masked_fill(nan, 0.0), want.masked_fill(nan, 0.0)) < 4e-3
+
+
+@pytest.mark.parametrize("T,hd", [(20, 128), (140, 64), (6, 128)])
+@pytest.mark.parametrize("scores", ["high", "low", "both"])
+@pytest.mark.parametrize("bad_value", [False, True])
+def test_attention_scores_near_the_largest(cuda_device, T, hd, scores, bad_value):
+    """Finite scores up to 3.3e38 in magnitude (times log2 e beyond fp32): differences are
+    taken before anything is scaled.  ``bad_value``: the last V row holds an infinity, which
+    takes the matrix form through its row-by-row branch and reaches the last query alone."""
+    from moeinfra_amd import _lib
+
+    nq, nkv, p0, max_seq = 4, 2, 500, 1024
+    S = p0 + T
+    q = torch.zeros((T, nq, hd), dtype=torch.bfloat16)
+    q[:, :, 0] = 1.0
+    k, v = _bf16((nkv, S, hd), 36), _bf16((nkv, S, hd), 37)
+    hot = torch.rand((nkv, S), generator=torch.Generator().manual_seed(8)) < 0.1
+    hot[:, 0] = True
+    top, rest = {"high": (3.3e38, 2.5e38), "low": (-2.5e38, -3.3e38), "both": (3.3e38, -3.3e38)}[scores]
+    k[:, :, 0] = torch.where(hot, top, rest).to(torch.bfloat16)
+    clean = v.clone()
+    if bad_value:
+        v[:, S - 1, 3] = float("inf")
+    kc = torch.zeros((nkv, max_seq, hd), dtype=torch.bfloat16)
+    vc = kc.clone()
+    kc[:, :S], vc[:, :S] = k, v
+    n = _lib.lib().moe_attention_workspace_bytes(T, nq, nkv, hd, max_seq)
+    ws = torch.zeros((max(n, 16),), dtype=torch.uint8, device=cuda_device)
+    want = _attend_ref(q, k, clean, p0, 1.0).reshape(T, nq, hd)
+    hit = torch.zeros((T, nq, hd), dtype=torch.bool)
+    hit[T - 1, :, 3] = bad_value
+    for w in (None, ws):
+        got = _attend(q.to(cuda_device), kc.to(cuda_device), vc.to(cuda_device), p0, w, 1.0)
+        got = got.cpu().float().reshape(T, nq, hd)
+        assert torch.isfinite(got[~hit]).all() and not torch.isfinite(got[hit]).any()
+        # As test_attention: bf16 rounding of the probabilities and of the output.
+        assert rel_l2(got.masked_fill(hit, 0.0), want.masked_fill(hit, 0.0)) < 4e-3
 
 
 @pytest.mark.parametrize("T,N,K", [(1, 6144, 4096), (1, 4096, 4096), (1, 1000, 512), (4, 515, 1024)])
