@@ -731,8 +731,8 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
   }
   if (nact > 1) {
     // Partial results to the workspace, word w of a lane at [w][lane] of its wave's block;
-    // the split that finishes a row tile last adds the others' to its own and writes the
-    // rows.
+    // the split that finishes a row tile last adds them up, in split order whichever it is
+    // (its own too is read back), and writes the rows.
     constexpr int kWords = (16 * kDT + 2) * kWave;
     const int unit = (int)blockIdx.x;
     float *const pu = part + ((size_t)unit * gridDim.y * 4 + wave) * kWords + lane;
@@ -748,8 +748,13 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
     }
     if (!attn_last_of(count + unit, nact)) return;  // uniform over the workgroup
     if (!live) return;
+    m = -INFINITY;
+    l = 0.0f;
+#pragma unroll
+    for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[dt][v] = 0.0f;
     for (int y = 0; y < nact; ++y) {
-      if (y == split) continue;
       const float *pw = pu + (size_t)y * 4 * kWords;
       const float m1 = attn_get(pw + 16 * kDT * kWave), l1 = attn_get(pw + (16 * kDT + 1) * kWave);
       const float mn = fmaxf(m, m1);

@@ -280,6 +280,30 @@ def test_attention_scores_near_the_largest(cuda_device, T, hd, scores, bad_value
         assert rel_l2(got.masked_fill(hit, 0.0), want.masked_fill(hit, 0.0)) < 4e-3
 
 
+@pytest.mark.parametrize("hd", [64, 128])
+def test_attention_splits_join_in_order(cuda_device, hd):
+    """The partial outputs of a row's key splits add up in split order, whichever workgroup
+    finishes last.  With q = 0 every key has weight one; the first two splits (256 keys each)
+    sum to +-2^28 and cancel, the others to 8 each, which a sum that starts with one of them
+    (fp32: a unit of 32 at 2^28) loses."""
+    from moeinfra_amd import _lib
+
+    T, n, max_seq = 40, 8, 8192
+    p0 = max_seq - T
+    q = torch.zeros((T, n, hd), dtype=torch.bfloat16, device=cuda_device)
+    k = _bf16((n, max_seq, hd), 46).to(cuda_device)
+    v = torch.full((n, max_seq, hd), 2.0 ** -5, dtype=torch.bfloat16, device=cuda_device)
+    v[:, :256], v[:, 256:512] = 2.0 ** 20, -(2.0 ** 20)
+    ws = torch.zeros((_lib.lib().moe_attention_workspace_bytes(T, n, n, hd, max_seq),),
+                     dtype=torch.uint8, device=cuda_device)
+    keys = torch.arange(p0 + 1, max_seq + 1, device=cuda_device, dtype=torch.float32)
+    want = ((keys - 512) / 32 / keys)[:, None].expand(T, n * hd)
+    for _ in range(3):
+        got = _attend(q, k, v, p0, ws)
+        # one bf16 rounding (a lost split is 3.4 % off)
+        assert torch.allclose(got.float(), want, rtol=2.0 ** -8, atol=0.0)
+
+
 @pytest.mark.parametrize("T,N,K", [(1, 6144, 4096), (1, 4096, 4096), (1, 1000, 512), (4, 515, 1024)])
 def test_gemv(cuda_device, T, N, K):
     from moeinfra_amd import _lib
