@@ -361,7 +361,8 @@ combine_kernel(const float *__restrict__ ypart, int nsplit, int64_t rows_total,
     if (pos < 0 || pos >= rows_total) continue;
     const float w = wts[t * k + j];
     float4 y = *reinterpret_cast<const float4 *>(ypart + (size_t)pos * H + c);
-    const int np = RANGES ? planes[(size_t)pos * (H / cols) + c / cols] : nsplit;
+    // (At most the planes there are: the rows of an absent expert have no count.)
+    const int np = RANGES ? min((int)planes[(size_t)pos * (H / cols) + c / cols], nsplit) : nsplit;
 #pragma unroll 4
     for (int s = 1; s < np; ++s) {
       const float4 v = *reinterpret_cast<const float4 *>(ypart + s * split_stride + (size_t)pos * H + c);
@@ -402,7 +403,7 @@ __global__ void reduce_splits_kernel(const float *__restrict__ ypart, int nsplit
   if (i >= numel) return;
   float4 acc = *reinterpret_cast<const float4 *>(ypart + i);
   // Row i / H's items follow each other in `planes`, cols columns each (H a multiple).
-  const int np = RANGES ? planes[i / cols] : nsplit;
+  const int np = RANGES ? min((int)planes[i / cols], nsplit) : nsplit;
   for (int s = 1; s < np; ++s) {
     const float4 v = *reinterpret_cast<const float4 *>(ypart + (size_t)s * numel + i);
     acc.x += v.x;

@@ -641,6 +641,31 @@ def test_down_in_ranges(cuda_device, T, k, E, H, F, skew):
     assert (out != want).float().mean() < 0.1
 
 
+def test_down_in_ranges_absent_expert(cuda_device):
+    """Rows of an absent expert have no item, so nothing writes their piece counts: whatever
+    byte is there, the combine stays within the planes that the workspace has.  (Zero planes,
+    counts of 255, and behind them, inside one large buffer, values that must not be read.)"""
+    from moeinfra_amd import _lib, ops
+    from moeinfra_amd._lib import MoeNf4Expert
+
+    T, k, E, H, F = 300, 2, 8, 1024, 3584
+    g = torch.Generator(device=cuda_device).manual_seed(5)
+    keep = [{n: ops.nf4_quantize((torch.randn(s, generator=g, device=cuda_device) * 0.02).to(torch.bfloat16))
+             for n, s in (("w1", (F, H)), ("w3", (F, H)), ("w2", (H, F)))} for _ in range(E - 1)]
+    some = [MoeNf4Expert(*(t.data_ptr() for n in ("w1", "w3", "w2") for t in st[n])) for st in keep]
+    table = ops.expert_table(some + [None])          # the last expert's rows are the last rows
+    gate = (torch.randn((E, H), generator=g, device=cuda_device) * 0.02).to(torch.bfloat16)
+    x = torch.randn((T, H), generator=g, device=cuda_device).to(torch.bfloat16)
+    need = _lib.lib().moe_layer_workspace_bytes(T, k, E, H, F)
+    plane = T * k * H * 4
+    ws = torch.full((need + 255 * plane,), 255, dtype=torch.uint8, device=cuda_device)
+    ws[:need] = 0
+    ws[need - T * k * H // 512:need] = 255           # the piece counts end the workspace
+    out, _, _, idx = ops.layer_forward(table, E, gate, x, k, F, workspace=ws)
+    assert (idx == E - 1).any() and torch.isfinite(out.float()).all()
+    assert (ws[need:] == 255).all()
+
+
 @pytest.mark.parametrize("T,k,E,H,F", [
     (13, 2, 8, 1024, 3584),     # seven K splits of the down projection, gate/up K-split
     (9, 2, 4, 512, 1536),       # three
