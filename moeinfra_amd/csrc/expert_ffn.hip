@@ -597,7 +597,12 @@ int launch_expert_ffn(const moe_nf4_expert_t *experts, int32_t E, const void *x,
   const int64_t wg_cap = (int64_t)device_cu_count() * 2;
   const int mt = token_tiles_for(max_tokens_per_expert);
 
-  if (nsplit == 1 && gemv4_chosen(max_tokens_per_expert, E, H, F))
+  // A lone expert's down projection leaves the GEMV only with the plane count of the form that
+  // takes its place: in one plane that form has a few workgroups (H = 4096, 1024, 4 tokens:
+  // 88 and 27 us, 26 and 13 with the GEMV).
+  const bool lone_planes = (phases & 2) && nsplit != choose_nsplit(max_tokens_per_expert, 1, E, H, F);
+  if (nsplit == 1 && (gemv4_chosen(max_tokens_per_expert, E, H, F) ||
+                      (E == 1 && lone_planes && gemv4_supported(max_tokens_per_expert, H, F))))
     return launch_gemv4(&tab, x, H, F, &rt, h_ws, ypart, phases, active_max, rows_total, fused,
                         stream);
   // Mid-size batches (up to 64 tokens): gate/up on 16-row weight tiles of "virtual experts"

@@ -702,3 +702,30 @@ def test_lone_expert_few_tokens(cuda_device, T, H, F):
     want = orc.bf16_to_f32(orc.swiglu(bits(x), *expert.dequant_np()))
     got = ops.expert_swiglu(expert.to(cuda_device).c_struct(), x.to(cuda_device), H, F)
     assert orc.rel_l2(orc.bf16_to_f32(bits(got)), want) <= 1e-2
+
+
+@pytest.mark.parametrize("T", [1, 4])
+@pytest.mark.parametrize("H,F", [(4096, 4096), (1024, 3584)])
+def test_lone_expert_separate_calls(cuda_device, T, H, F):
+    """The separate calls of one expert with one plane run the GEMV, as an expert among others
+    does: the same bits as a table of two experts with every token on the first (the forms
+    that the whole call of a lone expert takes are made for their own plane counts)."""
+    from moeinfra_amd import _lib, ops
+    from moeinfra_amd._lib import MoeNf4Expert
+
+    g = torch.Generator(device=cuda_device).manual_seed(T + F)
+    st = {n: ops.nf4_quantize((torch.randn(s, generator=g, device=cuda_device) * 0.02).to(torch.bfloat16))
+          for n, s in (("w1", (F, H)), ("w3", (F, H)), ("w2", (H, F)))}
+    ex = MoeNf4Expert(*(t.data_ptr() for n in ("w1", "w3", "w2") for t in st[n]))
+    x = torch.randn((T, H), generator=g, device=cuda_device).to(torch.bfloat16)
+    zero = torch.zeros((T, 1), dtype=torch.int32, device=cuda_device)
+    assert ops.choose_nsplit(T, 1, 2, H, F) == 1
+    got = [ops.expert_ffn(ops.expert_table([ex] * E), E, x, 1, H, F, ops.permute(zero, E), nsplit=1)
+           for E in (1, 2)]
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    # the down projection by itself, from the same h
+    route, y = ops.permute(zero, 1), torch.empty_like(got[1][1])
+    _lib.check(_lib.lib().moe_expert_down_nf4(
+        ops.expert_table([ex]), 1, T, 1, H, F, *(route[n].data_ptr() for n in ("counts", "offsets", "perm_tok", "active")),
+        got[1][0].data_ptr(), y.data_ptr(), 1, torch.cuda.current_stream().cuda_stream), "down")
+    assert torch.equal(y, got[1][1])
