@@ -480,13 +480,15 @@ int launch_mid_gateup(const void *tab, const void *x, int64_t T, int32_t k, int3
                       const void *route_out);
 
 // Up to 4 tokens per expert run the 4x4x4 MFMA GEMV.  A lone expert does not where the mid-size
-// kernels or the K-split items take its shape: the GEMV's work grows with the tokens and one
-// expert's rows do not fill the chip with it (H = 4096, F = 14336, 1 / 2 / 4 tokens: 48 / 52 /
-// 64 us a call, 43 / 44 / 44 with the mid-size kernels; H = 3072: 36 / 39 / 47 and 36 / 36 /
-// 37; layers of 16 experts are 4 % faster with it).
+// kernels or, from 2 tokens on, the K-split items take its shape: the GEMV's work grows with
+// the tokens and one expert's rows do not fill the chip with it (H = 4096, F = 14336, 1 / 2 /
+// 4 tokens: 46 / 49 / 61 us a call, 42 / 42 / 43 with the mid-size kernels; H = 3072, F = 8192,
+// K-split items: 34 / 37 / 46 and 36 / 37 / 38; H = 1024: 26 / 27 / 30 and 26 / 26 / 27; layers
+// of 16 experts are 4 % faster with it).
 bool gemv4_chosen(int64_t max_tokens, int32_t E, int32_t H, int32_t F) {
   return gemv4_supported(max_tokens, H, F) &&
-         !(E == 1 && (mid_gateup_supported(max_tokens, 1, 1, H, F) || midbatch_supported(H, F, 1)));
+         !(E == 1 && (mid_gateup_supported(max_tokens, 1, 1, H, F) ||
+                      (max_tokens > 1 && midbatch_supported(H, F, 1))));
 }
 
 // ypart planes a layer's down projection writes (the combine adds them): the streamed

@@ -71,6 +71,16 @@ def test_down_splits_size_the_ypart_planes():
         assert ws >= n * T * k * H * 4 + T * k * F * 2
 
 
+def test_lone_expert_leaves_the_gemv_from_two_tokens():
+    # One plane: the GEMV (34 us at hidden 3072 where the K-split items take 36).  At hidden
+    # 2048 and 4096 the mid-size kernels take one token too.
+    lib = _lib.lib()
+    for H, F in ((3072, 8192), (1024, 3584)):
+        assert lib.moe_layer_down_splits(1, 1, 1, H, F) == 1
+        assert lib.moe_layer_down_splits(2, 1, 1, H, F) > 1
+    assert lib.moe_layer_down_splits(1, 1, 1, 4096, 14336) == 7
+
+
 @pytest.mark.parametrize("call,needle", [
     (lambda l: l.moe_nf4_dequant_bf16(8, 8, 8, 8, 7, 64, None), "even"),
     (lambda l: l.moe_nf4_dequant_bf16(8, 8, 8, 8, 64, 48, None), "multiple of 32"),
