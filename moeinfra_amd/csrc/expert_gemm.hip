@@ -167,10 +167,14 @@ __device__ __forceinline__ uint16_t gm_swiglu_bf16(float g, float u) {
 constexpr int kMaxRanges = 512;  // workgroups of a launch
 constexpr int kMinPiece = 2;     // units: a shorter piece costs more than it evens out
 
-// Cost of a block of an item with `live` 32-token tiles of MT, in twentieths of a full one.
+// Cost of a block of an item with `live` 32-token tiles of MT, in twentieths of a full one
+// (fitted to 686 timed layers: a unit of 4 blocks takes 2.9 us and 0.36 us a live tile.  With
+// 8 + 12 live / MT the workgroups with partial items got too much of the work: against whole K
+// splits, a skewed layer of 180 / 512 / 800 tokens was 4.7 / 0.5 / 2.8 % slower in ranges and is
+// 2.9 / 5.4 / 4.0 % faster so; even routings of 512 / 1500: 2.3 / 3.1 % faster, now 4.9 / 6.1 %).
 template <int MT, bool PIPE>
 __device__ __forceinline__ int gm_cost(int live) {
-  return PIPE ? (2 * live <= MT ? 13 : 20) : live >= MT ? 20 : 8 + 12 * live / MT;
+  return PIPE ? (2 * live <= MT ? 13 : 20) : live >= MT ? 20 : 14 + 6 * live / MT;
 }
 
 // s_bound[v]: first unit of workgroup v's range, v <= G.  An item meets at most `planes`
