@@ -80,21 +80,15 @@ struct LayerWs {
   int64_t idx32, counts, offsets, perm_tok, slot_pos, active, counter, droute, h, ypart,
       ypart_bytes, pieces, total;
   int nsplit;
-  int cols;  // > 0: the down projection runs in ranges, `pieces` bytes per item of cols columns
+  int cols;  // > 0: the down projection counts its items' planes, a byte per row and cols columns
 };
 
 // one_plane: a single ypart plane instead of the default number.
 LayerWs layer_ws(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, bool one_plane = false) {
   LayerWs w{};
   const int64_t rows = T * k;
-  int planes = choose_nsplit(T, k, E, H, F);
-  w.nsplit = one_plane ? 1 : planes;
   const int ranges = one_plane ? 0 : layer_range_planes(T, k, E, H, F, &w.cols);
-  if (ranges > 0) {
-    w.nsplit = ranges;
-    planes = ranges > planes ? ranges : planes;
-  }
-  if (one_plane) planes = 1;
+  w.nsplit = one_plane ? 1 : ranges > 0 ? ranges : choose_nsplit(T, k, E, H, F);
   int64_t o = 0;
   w.idx32 = o;    o = align_up(o + rows * 4);
   w.counts = o;   o = align_up(o + (int64_t)E * 4);
@@ -105,7 +99,7 @@ LayerWs layer_ws(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, bool one
   w.counter = o;  o = align_up(o + 4);
   w.droute = o;   o = align_up(o + decode_route_bytes());
   w.h = o;        o = align_up(o + rows * (int64_t)F * 2);
-  w.ypart = o;    o = align_up(o + (int64_t)planes * rows * H * 4);
+  w.ypart = o;    o = align_up(o + (int64_t)w.nsplit * rows * H * 4);
   w.ypart_bytes = o - w.ypart;
   w.pieces = o;   o = align_up(o + (w.cols > 0 ? rows * (H / w.cols) : 0));
   w.total = o;

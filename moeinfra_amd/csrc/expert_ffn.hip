@@ -507,8 +507,9 @@ int choose_nsplit(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F) {
   return midbatch_splits(active_max, H, F);
 }
 
-// ypart planes of a layer (T tokens, k slots, E experts) whose down projection runs in ranges
-// on the batched GEMM, and its output columns per item; 0 for other layers.
+// ypart planes of a layer (T tokens, k slots, E experts) whose down projection may run in
+// ranges on the batched GEMM, or in the K splits of choose_nsplit where the routed counts make
+// those the better cut, and its output columns per item; 0 for other layers.
 int layer_range_planes(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, int *cols) {
   const int64_t rows = T * k;
   const int64_t active_max = rows < E ? rows : E;
@@ -517,7 +518,8 @@ int layer_range_planes(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F, in
       !expert_gemm_rows_ok(T, rows, H, F) || !expert_gemm_ranges_ok(rows, active_max, H, F))
     return 0;
   *cols = expert_gemm_down_cols(rows, active_max);
-  return expert_gemm_planes(rows, active_max, H, F);
+  const int ranges = expert_gemm_planes(rows, active_max, H, F), splits = expert_gemm_splits(rows, active_max, H, F);
+  return ranges > splits ? ranges : splits;
 }
 
 bool mid_layer_supported(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F);

@@ -158,11 +158,12 @@ __device__ __forceinline__ uint16_t gm_swiglu_bf16(float g, float u) {
 // the items are laid end to end, weighted by what a block of each costs (a partial token
 // tile skips MFMAs but not its weights), and cut into one equal range per workgroup, at
 // 4-block units.  An item cut by range ends has its pieces in successive planes, most items
-// are whole or in two pieces, and the sum reads the planes that an item has.  The cuts depend
-// on the routed counts alone, so results repeat bit for bit.  Down + sum over the
-// planes, 512 tokens: 274 + 25 -> 239 + 14 us; a layer of 512 / 900 / 1500 tokens 612 -> 598,
-// 838 -> 806, 1313 -> 1281 us; hidden 1024 at 300 tokens (32 K-split items before) 108 -> 86;
-// one expert of 128 tokens 203 -> 183 us.  Not for gate/up, whose pieces would have to meet
+// are whole or in two pieces, and the sum reads the planes that an item has.  The cuts, and
+// whether the K splits are the better ones after all, depend on the routed counts alone, so
+// results repeat bit for bit.  A layer of 512 / 900 / 1500 tokens, K splits and so: 612 -> 580,
+// 837 -> 791, 1321 -> 1235 us, with skewed routing 571 -> 541, 867 -> 802, 1313 -> 1225; hidden
+// 1024 at 300 tokens (32 K-split items before) 105 -> 82; one expert of 128 tokens 187 -> 170.
+// Choosing from the counts takes 1 to 2 us.  Not for gate/up, whose pieces would have to meet
 // before the SwiGLU: 256 KB of fp32 sums a piece cost a CU about what the round saves.
 constexpr int kMaxRanges = 512;  // workgroups of a launch
 constexpr int kMinPiece = 2;     // units: a shorter piece costs more than it evens out
@@ -176,46 +177,93 @@ template <int MT, bool PIPE>
 __device__ __forceinline__ int gm_cost(int live) {
   return PIPE ? (2 * live <= MT ? 13 : 20) : live >= MT ? 20 : 14 + 6 * live / MT;
 }
+// What a piece costs besides its blocks (first loads, fp32 stores): 10 us, in the same unit.
+constexpr int kPieceCost = 45;
 
-// s_bound[v]: first unit of workgroup v's range, v <= G.  An item meets at most `planes`
-// ranges: a range holds at least 1 / (planes - 1) of the dearest item's cost.
-template <int MT, bool PIPE>
-__device__ __forceinline__ void gm_bounds(const int (*s_ex)[5], int *s_bound, int n_active, int n_items,
-                                          int wtiles, int U, int G, int planes, int tid, int threads) {
-  // Per expert: cost of one weight tile's token tiles, and of its last (partial) one.
-  auto last_cost = [&](int a) { return gm_cost<MT, PIPE>((s_ex[a][1] - 32 * MT * (s_ex[a][4] - 1) + 31) >> 5); };
-  auto col_cost = [&](int a) { return s_ex[a][4] > 0 ? 20 * (s_ex[a][4] - 1) + last_cost(a) : 0; };
-  uint64_t total = 0;
-  int dear = 1;  // cost of a block of the dearest item
-  for (int a = 0; a < n_active; ++a) {
-    total += (uint64_t)col_cost(a) * (uint64_t)(wtiles * U);
-    dear = max(dear, s_ex[a][4] > 1 ? 20 : s_ex[a][4] == 1 ? last_cost(a) : 0);
+// The routed counts as the cuts below see them: per active expert s_ex (id, rows, row offset,
+// first item, token tiles) and s_cut (cost of the experts before it, cost of a block of its
+// last token tile), and s_sum: the cost of all items, of a block of the dearest item.
+struct GmCounts {
+  const int (*ex)[5];
+  const int (*cut)[2];
+  const int *sum;
+  int n_active;
+  // Active index of piece p of ks to an item: the last whose first piece is not beyond p (the
+  // experts without items before it start at the same piece).
+  __device__ __forceinline__ int of_piece(int p, int ks) const {
+    int a = -1;
+#pragma unroll 8
+    for (int j = 0; j < n_active; ++j) a += ex[j][3] * ks <= p ? 1 : 0;
+    return a;
   }
-  const uint64_t most = total * (uint64_t)max(planes - 1, 1) / (uint64_t)(dear * U);
-  const int ways = most < 1 ? 1 : most < (uint64_t)G ? (int)most : G;
+  __device__ __forceinline__ int cost(int p, int ks) const {
+    const int a = of_piece(p, ks), mtiles = ex[a][4];
+    return (p - ex[a][3] * ks) % mtiles < mtiles - 1 ? 20 : cut[a][1];
+  }
+};
+
+// How many ranges: one per workgroup, but an item meets at most `planes` of them, so a range
+// holds at least 1 / (planes - 1) of the dearest item's cost.  32 bits hold every cost here: h
+// of the launch is below 2^31 bytes, so its units are below 2^21 and their cost below 2^26.
+__device__ __forceinline__ int gm_ways(const GmCounts &c, int U, int G, int planes) {
+  return min(max(c.sum[0] * max(planes - 1, 1) / (c.sum[1] * U), 1), G);
+}
+
+// s_bound[v]: first unit of workgroup v's range, v <= G.
+__device__ __forceinline__ void gm_bounds(const GmCounts &c, int *s_bound, int n_items, int wtiles, int U, int G,
+                                          int ways, int tid, int threads) {
+  const int each = c.sum[0] / ways, over = c.sum[0] - each * ways;
   for (int i = tid; i <= G; i += threads) {
     int b = n_items * U;
     if (i < ways) {
-      uint64_t pos = total * (uint64_t)i / (uint64_t)ways;
-      int a = 0;
-      for (; a < n_active - 1; ++a) {
-        const uint64_t c = (uint64_t)col_cost(a) * (uint64_t)(wtiles * U);
-        if (pos < c) break;
-        pos -= c;
-      }
-      const int cu = col_cost(a) * U;
-      if (cu > 0) {
-        const int wt = min((int)(pos / (uint64_t)cu), wtiles - 1);
-        const int r = (int)(pos - (uint64_t)wt * (uint64_t)cu);
-        const int mt = min(r / (20 * U), s_ex[a][4] - 1);
-        int u = (r - mt * 20 * U) / (mt == s_ex[a][4] - 1 ? last_cost(a) : 20);
-        u = min(u, U);
-        u = u < kMinPiece ? 0 : u > U - kMinPiece ? U : u;
-        b = (s_ex[a][3] + wt * s_ex[a][4] + mt) * U + u;
-      }
+      const int pos = each * i + over * i / ways;  // total * i / ways
+      int a = -1;
+#pragma unroll 8
+      for (int j = 0; j < c.n_active; ++j) a += c.cut[j][0] <= pos ? 1 : 0;
+      const int mtiles = c.ex[a][4], last = c.cut[a][1];
+      const int col = (20 * (mtiles - 1) + last) * U;  // a weight tile's token tiles
+      const int wt = min((pos - c.cut[a][0]) / col, wtiles - 1);
+      const int r = pos - c.cut[a][0] - wt * col;
+      const int mt = min(r / (20 * U), mtiles - 1);
+      int u = min((r - mt * 20 * U) / (mt == mtiles - 1 ? last : 20), U);
+      u = u < kMinPiece ? 0 : u > U - kMinPiece ? U : u;
+      b = (c.ex[a][3] + wt * mtiles + mt) * U + u;
     }
     s_bound[i] = b;
   }
+}
+
+// Whether to take `ways` ranges or `ks` K splits of every item dealt out one by one: the one
+// whose longest workgroup ends first, by the same costs.  Splits that make one round need no
+// look at the workgroups (one that finds a whole item's split sets the time), and the ranges
+// have to be 10 % shorter, as those splits have no more planes and share an expert's weights in
+// L2: 16 experts, hidden 2048, 450 tokens: 269 us in splits, 278 in ranges of the same length.
+// Over more rounds ranges may be 4 % longer, for the planes that they save.
+__device__ __forceinline__ bool gm_ranges_beat_one_round(const GmCounts &c, int U, int ways, int ks) {
+  return 100 * (c.sum[0] / ways + kPieceCost) <= 90 * (U / ks * c.sum[1] + kPieceCost);
+}
+__device__ __forceinline__ bool gm_ranges_pay(const GmCounts &c, const int *s_bound, int *s_longest, int n_items,
+                                              int U, int G, int ks, int tid, int threads) {
+  float longest[2] = {0.0f, 0.0f};
+  for (int v = tid; v < G; v += threads) {
+    int sum = 0;
+    for (int u = s_bound[v]; u < s_bound[v + 1];) {
+      const int item = u / U, stop = min(s_bound[v + 1], (item + 1) * U);
+      sum += (stop - u) * c.cost(item, 1) + kPieceCost;
+      u = stop;
+    }
+    longest[0] = fmaxf(longest[0], (float)sum);
+    sum = 0;
+    for (int p = v; p < n_items * ks; p += G) sum += U / ks * c.cost(p, ks) + kPieceCost;
+    longest[1] = fmaxf(longest[1], (float)sum);
+  }
+  lane_groups_reduce<true>(longest, kWave);
+  if ((tid & (kWave - 1)) == 0) {
+    atomicMax(&s_longest[0], (int)longest[0]);
+    atomicMax(&s_longest[1], (int)longest[1]);
+  }
+  __syncthreads();
+  return 100 * (int64_t)s_longest[0] <= 104 * (int64_t)s_longest[1];
 }
 
 // The DMA's inline asm names M0, a register the compiler reserves and sets before each of
@@ -232,7 +280,7 @@ __global__ void __launch_bounds__(W * 64, 1)
 expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint32_t act_bytes,
                    int K, int NROWS, Route rt, int rows_total, int nsplit,
                    uint16_t *__restrict__ h_out, float *__restrict__ y_out,
-                   uint8_t *__restrict__ planes) {
+                   uint8_t *__restrict__ planes, int range_planes) {
   constexpr int kGmThreads = W * kWave;
   constexpr int kGmMT = MT;                            // 32-token MFMA tiles per item
   constexpr int kGmM = 32 * MT;                        // tokens per item
@@ -287,8 +335,10 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
   // (counted over the item), in place of a barrier per block.
   __shared__ int s_rdone;
   // Down with `planes` (see gm_bounds): workgroup v takes the 4-block units [s_bound[v],
-  // s_bound[v + 1]) of the items laid end to end.
+  // s_bound[v + 1]) of the items laid end to end, unless `nsplit` K splits of each item are
+  // the better cut (gm_ranges_pay).
   __shared__ int s_bound[GATEUP ? 1 : kMaxRanges + 1];
+  __shared__ int s_cut[GATEUP ? 1 : MOE_MAX_EXPERTS][2], s_sum[2], s_longest[2];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -310,7 +360,7 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
       // An absent expert (null pointers) gets no items; the caller routes no token to it.
       cnt = (GATEUP ? tab.e[e].w1_packed : tab.e[e].w2_packed) != nullptr ? rt.counts[e] : 0;
       mtiles = (cnt + kGmM - 1) / kGmM;
-      items = mtiles * (planes != nullptr ? 1 : nsplit) * wtiles;
+      items = mtiles * wtiles;
     }
     int incl = items;
 #pragma unroll
@@ -338,6 +388,27 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
       }
     }
     if (lane == kWave - 1) s_nitems = incl;
+    if (!GATEUP && planes != nullptr) {
+      const int last = gm_cost<MT, kPipe>((cnt - kGmM * (mtiles - 1) + 31) >> 5);
+      const int all = mtiles > 0 ? (20 * (mtiles - 1) + last) * wtiles * (NB >> 2) : 0;
+      int upto = all;
+      float dear[1] = {mtiles > 1 ? 20.0f : mtiles == 1 ? (float)last : 0.0f};
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        const int v = __shfl_up(upto, o);
+        if (lane >= o) upto += v;
+      }
+      lane_groups_reduce<true>(dear, kWave);
+      if (lane < n_active) {
+        s_cut[lane][0] = upto - all;
+        s_cut[lane][1] = last;
+      }
+      if (lane == kWave - 1) {
+        s_sum[0] = upto;
+        s_sum[1] = (int)dear[0];
+        s_longest[0] = s_longest[1] = 0;
+      }
+    }
   }
   for (int i = tid; i < n_active * 32; i += kGmThreads) {
     const moe_nf4_expert_t &ex = tab.e[rt.active[1 + (i >> 5)]];
@@ -370,30 +441,40 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
   // consecutive items [x G/8, (x + 1) G/8) of every round.
   const int vb = (G & 7) == 0 ? (int)(blockIdx.x & 7) * (G >> 3) + (int)(blockIdx.x >> 3)
                               : (int)blockIdx.x;
-  const bool ranges = !GATEUP && planes != nullptr;
+  bool ranges = false;
   const int U = NB >> 2;  // units per item
   int unit = 0, unit_end = 0;
+  if (!GATEUP && planes != nullptr && n_items > 0) {
+    const GmCounts counts{s_ex, s_cut, s_sum, n_active};
+    const int ways = gm_ways(counts, U, G, range_planes);
+    const bool one_round = n_items * nsplit <= G;
+    if (!one_round || gm_ranges_beat_one_round(counts, U, ways, nsplit)) {
+      gm_bounds(counts, s_bound, n_items, wtiles, U, G, ways, tid, kGmThreads);
+      __syncthreads();
+      ranges = one_round || gm_ranges_pay(counts, s_bound, s_longest, n_items, U, G, nsplit, tid, kGmThreads);
+    }
+  }
+  const int ks = ranges ? 1 : nsplit;
+  const int n_pieces = n_items * ks;
   if (ranges) {
-    gm_bounds<MT, kPipe>(s_ex, s_bound, n_active, n_items, wtiles, U, G, nsplit, tid, kGmThreads);
-    __syncthreads();
     unit = __builtin_amdgcn_readfirstlane(s_bound[vb]);
     unit_end = __builtin_amdgcn_readfirstlane(s_bound[vb + 1]);
     if (unit >= unit_end) return;  // uniform over the workgroup
-  } else if (vb >= n_items) {
+  } else if (vb >= n_pieces) {
     return;  // uniform over the workgroup
   }
 
   auto ex_field = [&](int a, int f) { return __builtin_amdgcn_readfirstlane(s_ex[a][f]); };
-  // Item -> (active index, weight tile, split, token tile); wave-uniform.
+  // Piece (with ks = 1: item) -> (active index, weight tile, split, token tile); wave-uniform.
   auto decode = [&](int item, int &a, int &wt, int &sp, int &mt) {
     const int sel = lane < n_active ? lane : 0;
-    a = __popcll(__ballot(lane < n_active && s_ex[sel][3] <= item)) - 1;
-    int rem = item - ex_field(a, 3);
+    a = __popcll(__ballot(lane < n_active && s_ex[sel][3] * ks <= item)) - 1;
+    int rem = item - ex_field(a, 3) * ks;
     const int mtiles = ex_field(a, 4);
     const int q = rem / mtiles;
     mt = rem - q * mtiles;
-    wt = planes != nullptr ? q : q / nsplit;
-    sp = planes != nullptr ? 0 : q - wt * nsplit;
+    wt = q / ks;
+    sp = q - wt * ks;
   };
 
   // Replica of the lane's table lookups per fragment: with one codebook in the table, lanes
@@ -727,9 +808,10 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
       }
     }
   };
-  for (int item = vb; ranges ? unit < unit_end : item < n_items; item += G) {
+  for (int item = vb; ranges ? unit < unit_end : item < n_pieces; item += G) {
     int a, wt, sp, mt;
     int kb0i, nb;  // blocks kb0i .. kb0i + nb - 1 of the item's K range
+    int n = ks;    // pieces of the item
     if (ranges) {
       item = unit / U;
       const int lo = item * U, stop = min(unit_end, lo + U);
@@ -742,18 +824,17 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
         auto bound = [&](int v) { return __builtin_amdgcn_readfirstlane(s_bound[v]); };
         for (int v = vb; bound(v) > lo; --v) sp += bound(v) > bound(v - 1) ? 1 : 0;
       }
-      if (kb0i == 0) {
-        // The item's first piece says how many there are, for the sum over the planes.
-        int n = 1;
-        for (int v = vb + 1; v < G && s_bound[v] < lo + U; ++v) n += s_bound[v + 1] > s_bound[v] ? 1 : 0;
-        const int rows = min(kGmM, ex_field(a, 1) - mt * kGmM);
-        for (int r = tid; r < rows; r += kGmThreads)
-          planes[(size_t)(ex_field(a, 2) + mt * kGmM + r) * wtiles + wt] = (uint8_t)n;
-      }
+      for (int v = vb + 1; v < G && s_bound[v] < lo + U; ++v) n += s_bound[v + 1] > s_bound[v] ? 1 : 0;
     } else {
       decode(item, a, wt, sp, mt);
       kb0i = sp * NBp;
       nb = NBp;
+    }
+    if (!GATEUP && planes != nullptr && kb0i == 0) {
+      // The item's first piece says how many there are, for the sum over the planes.
+      const int rows = min(kGmM, ex_field(a, 1) - mt * kGmM);
+      for (int r = tid; r < rows; r += kGmThreads)
+        planes[(size_t)(ex_field(a, 2) + mt * kGmM + r) * wtiles + wt] = (uint8_t)n;
     }
     if (kPipe && ex_field(a, 1) - mt * kGmM <= kGmM / 2)
       piece(a, wt, sp, mt, kb0i, nb, std::integral_constant<int, kPipe ? MT / 2 : MT>{});
@@ -824,18 +905,20 @@ int expert_gemm_splits(int64_t rows, int64_t active, int32_t H, int32_t F) {
 template <int W, int MT, int NF, int BD>
 static int launch_gemm_shape(const ExpertTable &tab, const void *x, int64_t T, int64_t rows_total,
                              int32_t H, int32_t F, const Route &rt, void *h_ws, void *ypart,
-                             int32_t nsplit, int phases, uint8_t *planes, hipStream_t stream) {
+                             int32_t nsplit, int phases, uint8_t *planes, int range_planes,
+                             hipStream_t stream) {
   const dim3 grid((unsigned)device_cu_count()), blk(W * kWave);
   if (phases & 1) {
     hipLaunchKernelGGL((expert_gemm_kernel<true, W, MT, NF, BD>), grid, blk, 0, stream, tab,
                        (const uint16_t *)x, (uint32_t)(T * H * 2), H, F, rt, (int)rows_total, 1,
-                       (uint16_t *)h_ws, (float *)nullptr, (uint8_t *)nullptr);
+                       (uint16_t *)h_ws, (float *)nullptr, (uint8_t *)nullptr, 0);
     MOE_LAUNCH_CHECK();
   }
   if (phases & 2) {
     hipLaunchKernelGGL((expert_gemm_kernel<false, W, MT, NF, BD>), grid, blk, 0, stream, tab,
                        (const uint16_t *)h_ws, (uint32_t)(rows_total * F * 2), F, H, rt,
-                       (int)rows_total, nsplit, (uint16_t *)nullptr, (float *)ypart, planes);
+                       (int)rows_total, nsplit, (uint16_t *)nullptr, (float *)ypart, planes,
+                       range_planes);
     MOE_LAUNCH_CHECK();
   }
   return MOE_STATUS_OK;
@@ -850,14 +933,16 @@ int expert_gemm_planes(int64_t rows, int64_t active, int32_t H, int32_t F) {
   const int64_t n = items > 0 ? (device_cu_count() + items - 1) / items + 2 : 1;
   return (int)(n < 2 ? 2 : n > 16 ? 16 : n);
 }
-// Whether a layer's down projection runs in ranges.  Not
+// Whether a layer's down projection may run in ranges (the kernel sees the routed counts and
+// decides).  Not
 //  * with 256-token items of four or more experts: 2 rounds of items or more, whose launch is
 //    bound by the clock that the chip's power allows, and items dealt out one by one share
 //    their operands in L2 (T = 4096: 2795 us a layer, 2930 in ranges; one expert of 2048
 //    tokens: 752 us in whole K splits, 667 in ranges);
 //  * where K splits fill every round for any routing near the average, through cheap planes
 //    (16 experts, top-4, hidden 2048, 300 tokens: 235 us, 250 in ranges, which start and end
-//    inside items).
+//    inside items), or fill one round to three quarters or more (one expert of 395 tokens:
+//    201 us, 204 in ranges; 16 experts, 380 tokens: 251 and 268).
 bool expert_gemm_ranges_ok(int64_t rows, int64_t active, int32_t H, int32_t F) {
   if (device_cu_count() > kMaxRanges || active < 1) return false;
   const GemmShape g = gemm_shape(rows, active);
@@ -870,7 +955,9 @@ bool expert_gemm_ranges_ok(int64_t rows, int64_t active, int32_t H, int32_t F) {
   const int64_t s = gemm_splits_for(g, rows, active, H, F);
   const int64_t pieces = active * ((per + m - 1) / m) * (H / g.down_rows()) * s;
   const int64_t rounds = (pieces + cus - 1) / cus;
-  return !(steady && 10 * pieces >= 9 * rounds * cus && s * rows * H * 4 <= (int64_t)40 << 20);
+  const int64_t plane_bytes = s * rows * H * 4;
+  if (steady && rounds == 1) return !(4 * pieces >= 3 * cus && plane_bytes <= (int64_t)72 << 20);
+  return !(steady && 10 * pieces >= 9 * rounds * cus && plane_bytes <= (int64_t)40 << 20);
 }
 int expert_gemm_down_cols(int64_t rows, int64_t active) { return (int)gemm_shape(rows, active).down_rows(); }
 
@@ -884,14 +971,25 @@ static int check_gemm_args(int64_t T, int64_t rows_total, int32_t H, int32_t F, 
 int launch_expert_gemm(const void *tab_v, const void *x, int64_t T, int64_t rows_total,
                        int64_t active_max, int32_t H, int32_t F, const void *route_v, void *h_ws,
                        void *ypart, int32_t nsplit, int phases, uint8_t *planes, hipStream_t stream) {
-  const int rc = check_gemm_args(T, rows_total, H, F, planes ? 1 : nsplit);
+  // With `planes`, `nsplit` is how many planes there are: enough for ranges and for the K
+  // splits that they are held against (layer_range_planes).
+  int range_planes = 0;
+  if (planes != nullptr) {
+    range_planes = expert_gemm_planes(rows_total, active_max, H, F);
+    const int splits = expert_gemm_splits(rows_total, active_max, H, F);
+    MOE_REQUIRE(nsplit >= range_planes && nsplit >= splits, "too few planes for the batched expert GEMM");
+    nsplit = splits;
+  }
+  const int rc = check_gemm_args(T, rows_total, H, F, nsplit);
   if (rc != MOE_STATUS_OK) return rc;
   const ExpertTable &tab = *static_cast<const ExpertTable *>(tab_v);
   const Route &rt = *static_cast<const Route *>(route_v);
   const GemmShape g = gemm_shape(rows_total, active_max);
   if (g.mt == 8)
-    return launch_gemm_shape<4, 8, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, planes, stream);
-  return launch_gemm_shape<8, 4, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, planes, stream);
+    return launch_gemm_shape<4, 8, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, planes,
+                                          range_planes, stream);
+  return launch_gemm_shape<8, 4, 2, 4>(tab, x, T, rows_total, H, F, rt, h_ws, ypart, nsplit, phases, planes,
+                                          range_planes, stream);
 }
 
 }  // namespace moe

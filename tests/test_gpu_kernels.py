@@ -616,7 +616,8 @@ def test_mid_down_needs_a_workgroup_per_pair(cuda_device):
 ])
 def test_down_in_ranges(cuda_device, T, k, E, H, F, skew):
     """A layer's down projection in ranges (items cut by equal shares of the work, their pieces
-    in as many ypart planes as each has) against the same layer through the separate calls,
+    in as many ypart planes as each has), or in the K splits that its counts make the better
+    cut, against the same layer through the separate calls,
     with whole items in one plane: fp32 sums in another order, so single bf16 roundings of
     the output differ (2^-9 of a value, on a small share of them)."""
     from moeinfra_amd import ops
@@ -639,6 +640,44 @@ def test_down_in_ranges(cuda_device, T, k, E, H, F, skew):
     want = ops.combine(ypart, w, idx32, route["slot_pos"])
     assert orc.rel_l2(out.float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-3
     assert (out != want).float().mean() < 0.1
+
+
+@pytest.mark.parametrize("hot", [True, False])
+def test_down_cut_follows_the_counts(cuda_device, hot):
+    """The down projection's cut is chosen from the routed counts.  Two experts with all the rows
+    (24 items, in 8 K splits one round of 192 workgroups): K splits.  Even rows (48 items, 384
+    pieces): ranges.  The piece counts at the workspace's end tell; the results agree with
+    whole items in one plane up to the order of fp32 sums."""
+    from moeinfra_amd import _lib, ops
+    from moeinfra_amd._lib import MoeNf4Expert
+
+    T, k, E, H, F = 130, 2, 8, 3072, 8192
+    g = torch.Generator(device=cuda_device).manual_seed(9)
+    st = {n: ops.nf4_quantize((torch.randn(s, generator=g, device=cuda_device) * 0.02).to(torch.bfloat16))
+          for n, s in (("w1", (F, H)), ("w3", (F, H)), ("w2", (H, F)))}
+    table = ops.expert_table([MoeNf4Expert(*(t.data_ptr() for n in ("w1", "w3", "w2") for t in st[n]))] * E)
+    # logits of +-1000: token t takes experts 0 and 1, or 2 (t % 4) and 2 (t % 4) + 1
+    t = torch.arange(T, device=cuda_device)
+    x = torch.randn((T, H), generator=g, device=cuda_device).to(torch.bfloat16)
+    x[:, :4] = 0.0
+    x[t, t % 4] = 1.0
+    gate = torch.zeros((E, H), dtype=torch.bfloat16, device=cuda_device)
+    pair = torch.arange(E, device=cuda_device) // 2
+    gate[:, :4] = torch.where(pair[:, None] == (0 if hot else torch.arange(4, device=cuda_device)[None, :]),
+                              1000.0, -1000.0).to(torch.bfloat16)
+    need = _lib.lib().moe_layer_workspace_bytes(T, k, E, H, F)
+    ws = torch.zeros((need,), dtype=torch.uint8, device=cuda_device)
+    out, _, w, idx = ops.layer_forward(table, E, gate, x, k, F, workspace=ws)
+    assert torch.bincount(idx.reshape(-1), minlength=E).tolist() == ([T, T] + [0] * 6 if hot else [33] * 4 + [32] * 4)
+    rows = T * k
+    pieces = ws[need - (rows * (H // 512) + 255) // 256 * 256:][:rows * (H // 512)]
+    assert (pieces == 8).all() if hot else (pieces > 0).all() and (pieces != 8).all()
+    idx32 = idx.to(torch.int32)
+    route = ops.permute(idx32, E)
+    _, ypart = ops.expert_ffn(table, E, x, k, H, F, route, nsplit=1)
+    want = ops.combine(ypart, w, idx32, route["slot_pos"])
+    # As test_down_in_ranges: single bf16 roundings differ.
+    assert orc.rel_l2(out.float().cpu().numpy(), want.float().cpu().numpy()) <= 1e-3
 
 
 def test_down_in_ranges_absent_expert(cuda_device):
