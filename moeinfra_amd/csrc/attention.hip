@@ -5,7 +5,8 @@
 //   attention_kernel          one workgroup per (query head, token), any head dim
 //   few_attention_kernel      up to 8 tokens: several workgroups share a row's keys
 //   prefill_attention_kernel  more tokens at head dim 64 or 128: 128 query rows per workgroup
-//                             on the matrix cores, one pass over the keys
+//                             on the matrix cores, one pass over the keys (a few dozen tokens
+//                             with a short context row by row)
 // Numbers below: 32 query heads, 8 KV heads of 128, MI355X, launches back to back.
 #include <type_traits>
 
@@ -62,15 +63,130 @@ __device__ __forceinline__ void attn_pv(const uint4 (&vv)[kAttnRowsInFlight], in
   }
 }
 
-// One workgroup per (query head, token): scores of keys 0 .. pos0 + t (causal), bf16 scores
-// scaled in bf16, fp32 softmax rounded to bf16, then the bf16 probabilities times V with
+// NH query heads of a KV head, one token, on kAttnThreads threads: scores of keys 0 .. pos0 + t
+// (causal), bf16 scores scaled in bf16, fp32 softmax rounded to bf16, then the bf16 probabilities times V with
 // fp32 accumulation.  A cache row of hd bf16 is read by hd/8 consecutive lanes, 16 bytes
-// each, so the workgroup covers rpp = 256/(hd/8) rows per load instruction and a pass takes
+// each, so the threads cover rpp = 256/(hd/8) rows per load instruction and a pass takes
 // 8 such loads per thread (128 rows at hd = 128); a score is the xor-shuffle sum over its
-// row's lanes.  The first pass's K and V rows are loaded together with q and the position,
-// before the key count is known (row indexes clamped to the cache, results of rows past the
-// last key discarded), so a context of up to one pass of keys costs one memory round trip;
-// later passes load rows clamped to the last key.
+// row's lanes.  The first pass's K and V rows are loaded together with q and the position
+// (first()), before the key count is known (row indexes clamped to the cache, results of rows
+// past the last key discarded), so a context of up to one pass of keys costs one memory round
+// trip; later passes load rows clamped to the last key.
+template <int NH>
+struct AttnRow {
+  const uint16_t *kbase, *vbase;
+  int tid, hd, lpr, rpp, sub, rr;
+  float qf[NH][8];
+  uint4 kv[kAttnRowsInFlight], vv[kAttnRowsInFlight];
+
+  __device__ __forceinline__ void load(uint4 (&dst)[kAttnRowsInFlight], const uint16_t *base, int j0, int last) {
+#pragma unroll
+    for (int u = 0; u < kAttnRowsInFlight; ++u)
+      dst[u] = *reinterpret_cast<const uint4 *>(base + (size_t)min(j0 + u * rpp + rr, last) * hd);
+  }
+  // Heads h .. h + NH - 1 of one KV head.
+  __device__ __forceinline__ void first(const uint16_t *q, const uint16_t *kc, const uint16_t *vc, int nq, int nkv,
+                                        int hd_, int64_t max_seq, int h, int t, int tid_) {
+    tid = tid_;
+    hd = hd_;
+    lpr = hd >> 3;               // lanes per row: a power of two <= 32
+    rpp = kAttnThreads / lpr;    // rows per load instruction
+    sub = tid & (lpr - 1);
+    rr = tid / lpr;
+#pragma unroll
+    for (int n = 0; n < NH; ++n)
+      unpack8(*reinterpret_cast<const uint4 *>(q + ((size_t)t * nq + h + n) * hd + sub * 8), qf[n]);
+    const int kvh = h / (nq / nkv);
+    kbase = kc + (size_t)kvh * max_seq * hd + sub * 8;
+    vbase = vc + (size_t)kvh * max_seq * hd + sub * 8;
+    load(kv, kbase, 0, (int)max_seq - 1);
+    load(vv, vbase, 0, (int)max_seq - 1);
+  }
+  // The NH output rows at `orow` over nkeys keys.  s_p: NH arrays of `stride` >= nkeys floats,
+  // s_red: NH per wave, s_acc: NH * kAttnThreads * 8.  The barriers are the same whatever nkeys is.
+  __device__ __forceinline__ void finish(int nkeys, float scaling, uint16_t *orow, float *s_p, int stride,
+                                         float *s_red, float *s_acc) {
+    constexpr int kWaves = kAttnThreads / kWave;
+    const int npass = kAttnRowsInFlight * rpp;
+    float mx[NH], sum[NH];
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+      mx[n] = -INFINITY;
+      attn_scores(kv, qf[n], 0, nkeys, rpp, rr, lpr, sub, scaling, s_p + n * stride, mx[n]);
+    }
+    for (int j0 = npass; j0 < nkeys; j0 += npass) {
+      load(kv, kbase, j0, nkeys - 1);
+#pragma unroll
+      for (int n = 0; n < NH; ++n)
+        attn_scores(kv, qf[n], j0, nkeys, rpp, rr, lpr, sub, scaling, s_p + n * stride, mx[n]);
+    }
+    // block max, then the block sum of the exponentials (each a wave reduction, then the
+    // four waves' values through LDS in wave order)
+    const int lane = tid & (kWave - 1), wave = tid >> 6;
+    lane_groups_reduce<true>(mx, kWave);
+    if (lane == 0)
+      for (int n = 0; n < NH; ++n) s_red[n * kWaves + wave] = mx[n];
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+      mx[n] = s_red[n * kWaves];
+      for (int w = 1; w < kWaves; ++w) mx[n] = fmaxf(mx[n], s_red[n * kWaves + w]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+      sum[n] = 0.0f;
+      for (int j = tid; j < nkeys; j += kAttnThreads) {
+        const float e = expf(s_p[n * stride + j] - mx[n]);
+        s_p[n * stride + j] = e;
+        sum[n] += e;
+      }
+    }
+    lane_groups_reduce<false>(sum, kWave);
+    if (lane == 0)
+      for (int n = 0; n < NH; ++n) s_red[n * kWaves + wave] = sum[n];
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+      sum[n] = 0.0f;
+      for (int w = 0; w < kWaves; ++w) sum[n] += s_red[n * kWaves + w];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < NH; ++n)
+      for (int j = tid; j < nkeys; j += kAttnThreads) s_p[n * stride + j] = bf16r(s_p[n * stride + j] / sum[n]);
+    __syncthreads();
+    // out[d] = sum_j p_j v_j[d]: thread (rr, sub) accumulates dims sub*8 .. sub*8+7 over rows
+    // rr, rr + rpp, ... in order; then the rpp partial rows are summed through LDS.
+    float acc[NH][8];
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[n][e] = 0.0f;
+      attn_pv(vv, 0, nkeys, rpp, rr, s_p + n * stride, acc[n]);
+    }
+    for (int j0 = npass; j0 < nkeys; j0 += npass) {
+      load(vv, vbase, j0, nkeys - 1);
+#pragma unroll
+      for (int n = 0; n < NH; ++n) attn_pv(vv, j0, nkeys, rpp, rr, s_p + n * stride, acc[n]);
+    }
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+      float4 *sa = reinterpret_cast<float4 *>(s_acc + n * kAttnThreads * 8 + rr * hd + sub * 8);
+      sa[0] = make_float4(acc[n][0], acc[n][1], acc[n][2], acc[n][3]);
+      sa[1] = make_float4(acc[n][4], acc[n][5], acc[n][6], acc[n][7]);
+    }
+    __syncthreads();
+    for (int i = tid; i < NH * hd; i += kAttnThreads) {
+      const int n = i / hd, d = i - n * hd;
+      float o = 0.0f;
+      for (int r = 0; r < rpp; ++r) o += s_acc[n * kAttnThreads * 8 + r * hd + d];
+      orow[i] = f32_to_bf16(o);
+    }
+  }
+};
+
+// One workgroup per (query head, token).
 __global__ void __launch_bounds__(kAttnThreads)
 attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc,
                  const uint16_t *__restrict__ vc, int nq, int nkv, int hd,
@@ -82,86 +198,11 @@ attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc
   MOE_ARGS_FIRST(MOE_LIST("+s"(nq), "+s"(nkv), "+s"(hd), "+s"(max_seq), "+s"(scaling)),
                  MOE_LIST("s"(q), "s"(kc), "s"(vc), "s"(pos0), "s"(out)));
   const int h = blockIdx.x, t = blockIdx.y;
-  const int kvh = h / (nq / nkv);
-  const int lpr = hd >> 3;               // lanes per row: a power of two <= 32
-  const int rpp = kAttnThreads / lpr;    // rows per load instruction of the workgroup
-  const int npass = kAttnRowsInFlight * rpp;
-  const int sub = threadIdx.x & (lpr - 1), rr = threadIdx.x / lpr;
-  float qf[8];
-  unpack8(*reinterpret_cast<const uint4 *>(q + ((size_t)t * nq + h) * hd + sub * 8), qf);
-  const uint16_t *kbase = kc + (size_t)kvh * max_seq * hd + sub * 8;
-  const uint16_t *vbase = vc + (size_t)kvh * max_seq * hd + sub * 8;
-  uint4 kv[kAttnRowsInFlight], vv[kAttnRowsInFlight];
-#pragma unroll
-  for (int u = 0; u < kAttnRowsInFlight; ++u) {
-    const int j = min(u * rpp + rr, (int)max_seq - 1);
-    kv[u] = *reinterpret_cast<const uint4 *>(kbase + (size_t)j * hd);
-    vv[u] = *reinterpret_cast<const uint4 *>(vbase + (size_t)j * hd);
-  }
+  AttnRow<1> row;
+  row.first(q, kc, vc, nq, nkv, hd, max_seq, h, t, (int)threadIdx.x);
   // Keys 0 .. pos0 + t, bounded by the cache (a position past it is a caller error).
-  const int nkeys = min(*pos0 + t + 1, (int)max_seq);
-  float mx = -INFINITY;
-  attn_scores(kv, qf, 0, nkeys, rpp, rr, lpr, sub, scaling, s_p, mx);
-  for (int j0 = npass; j0 < nkeys; j0 += npass) {
-#pragma unroll
-    for (int u = 0; u < kAttnRowsInFlight; ++u) {
-      const int j = min(j0 + u * rpp + rr, nkeys - 1);
-      kv[u] = *reinterpret_cast<const uint4 *>(kbase + (size_t)j * hd);
-    }
-    attn_scores(kv, qf, j0, nkeys, rpp, rr, lpr, sub, scaling, s_p, mx);
-  }
-  // block max, then the block sum of the exponentials (each a wave reduction, then the
-  // four waves' values through LDS in wave order)
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
-  {
-    float m[1] = {mx};
-    lane_groups_reduce<true>(m, kWave);
-    if (lane == 0) s_red[wave] = m[0];
-    __syncthreads();
-    mx = s_red[0];
-    for (int w = 1; w < kAttnThreads / kWave; ++w) mx = fmaxf(mx, s_red[w]);
-    __syncthreads();
-  }
-  float sum = 0.0f;
-  for (int j = threadIdx.x; j < nkeys; j += kAttnThreads) {
-    const float e = expf(s_p[j] - mx);
-    s_p[j] = e;
-    sum += e;
-  }
-  {
-    float v[1] = {sum};
-    lane_groups_reduce<false>(v, kWave);
-    if (lane == 0) s_red[wave] = v[0];
-    __syncthreads();
-    sum = 0.0f;
-    for (int w = 0; w < kAttnThreads / kWave; ++w) sum += s_red[w];
-    __syncthreads();
-  }
-  for (int j = threadIdx.x; j < nkeys; j += kAttnThreads) s_p[j] = bf16r(s_p[j] / sum);
-  __syncthreads();
-  // out[d] = sum_j p_j v_j[d]: thread (rr, sub) accumulates dims sub*8 .. sub*8+7 over rows
-  // rr, rr + rpp, ... in order; then the rpp partial rows are summed through LDS.
-  float acc[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-  attn_pv(vv, 0, nkeys, rpp, rr, s_p, acc);
-  for (int j0 = npass; j0 < nkeys; j0 += npass) {
-#pragma unroll
-    for (int u = 0; u < kAttnRowsInFlight; ++u) {
-      const int j = min(j0 + u * rpp + rr, nkeys - 1);
-      vv[u] = *reinterpret_cast<const uint4 *>(vbase + (size_t)j * hd);
-    }
-    attn_pv(vv, j0, nkeys, rpp, rr, s_p, acc);
-  }
-  float4 *sa = reinterpret_cast<float4 *>(s_acc + rr * hd + sub * 8);
-  sa[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-  sa[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
-  __syncthreads();
-  for (int d = threadIdx.x; d < hd; d += kAttnThreads) {
-    float o = 0.0f;
-    for (int r = 0; r < rpp; ++r) o += s_acc[r * hd + d];
-    out[((size_t)t * nq + h) * hd + d] = f32_to_bf16(o);
-  }
+  row.finish(min(*pos0 + t + 1, (int)max_seq), scaling, out + ((size_t)t * nq + h) * hd, s_p, 0, s_red,
+             s_acc);
 }
 
 // Partial results pass between workgroups, which may run on different XCDs, through
@@ -377,17 +418,24 @@ few_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict_
 // about 2.3 us (MFMA, score rounding and exponentials, and 256 KB of LDS operand reads a
 // pair), and 376 workgroups fill 256 CUs once and a half.  A second group of four waves takes
 // every other tile (the chain halves; their sums meet in LDS), and where row tiles alone
-// leave CUs idle, workgroups share a tile's keys through the workspace.  1500 tokens: 1025 us
-// one workgroup per (head, token), 42 us here; 500 tokens behind 2000: 978 and 41 us; 40
-// behind 2500: 102 and 26 us; 40 alone: 8.4 and 9.9 us (one pair of tiles is about 8 us from
-// end to end, which is why up to kFewTokens = 8 tokens keep the other form: 4.2 us at 7
-// tokens).
+// leave CUs idle, workgroups share a tile's keys through the workspace.  1500 tokens: 1022 us
+// one workgroup per (head, token), 40 us here; 500 tokens behind 2000: 967 and 39 us; 40
+// behind 2500: 99 and 24 us.
 // Key tiles wait in registers while the previous pair is multiplied; two LDS planes per key
 // group make that one barrier per pair.
+//
+// One pair of tiles is 8 to 10 us from end to end, most of it first use of the code and of the
+// loads, more than a row takes alone (up to kFewTokens = 8 tokens keep the other form: 4.2 us
+// at 7).  So a lone pair goes through group 0 without the joining of the groups (40 tokens: 9.9
+// -> 8.2 us; one workgroup per row 8.5), and up to kFaRowKeys keys, where the device holds all
+// units of ROWS heads of a token at once, the workgroups take those instead: 9 / 16 / 32 tokens
+// 7.9 / 8.4 / 9.8 us in pairs, 4.7 / 4.9 / 7.2 one workgroup per row, 4.4 / 4.5 / 6.3 so; 32
+// behind 100 / 300: 13.0 / 14.4, 9.6 / 17.2 and 9.4 / 13.3.
 constexpr int kFaThreads = 512;
 constexpr int kFaHalf = 256;  // threads of one key group
 constexpr int kFaRows = 128;  // query rows per workgroup
 constexpr int kFaKeys = 64;   // keys per tile
+constexpr int kFaRowKeys = 384;  // the row instance's keys at most
 constexpr float kLog2e = 1.44269504088896341f;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 
@@ -468,13 +516,13 @@ __device__ __forceinline__ void fa_load_row(const float *s_row, int row, int hh,
   l = src[HD + 1];
 }
 
-template <int HD>
+template <int HD, int ROWS>
 __global__ void __launch_bounds__(kFaThreads, 2)
 prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc,
                          const uint16_t *__restrict__ vc, int T, int nq, int nkv,
                          const int32_t *__restrict__ pos0, int64_t max_seq, float scaling,
                          uint16_t *__restrict__ out, uint32_t *__restrict__ count,
-                         float *__restrict__ part) {
+                         float *__restrict__ part, int splits) {
   static_assert(HD == 64 || HD == 128, "head dims of the matrix form");
   constexpr int kPieces = HD / 8;                       // 16-byte pieces per K row
   constexpr int kKRows = kFaHalf / kPieces;             // K rows per load instruction
@@ -483,6 +531,30 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
   constexpr int kDT = HD / 32;                          // 32-dim output tiles
   constexpr int kKPlane = kFaKeys * HD * 2, kVPlane = HD * kFaKeys * 2;  // bytes
   __shared__ __attribute__((aligned(16))) uint8_t s_kv[2][2][kKPlane + kVPlane];
+  __shared__ int s_nonfinite;
+
+  if constexpr (ROWS > 0) {
+    // Two units of ROWS heads of a token a workgroup.  (Their loads are on the way when the
+    // position arrives; a long context drops them.)
+    constexpr int kAcc = ROWS * kAttnThreads * 8, kUnit = kAcc + ROWS * (kFaRowKeys + kAttnThreads / kWave);
+    static_assert(2 * kUnit * 4 <= (int)sizeof(s_kv), "the units fit the planes");
+    const int half = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kAttnThreads);
+    const int wg = (int)(blockIdx.y * gridDim.x + blockIdx.x);
+    const int units = nq / ROWS * T;
+    const int unit = min(2 * wg + half, units - 1);  // (an odd last unit twice, the same values)
+    const int t = unit / (nq / ROWS), h = (unit - t * (nq / ROWS)) * ROWS;
+    AttnRow<ROWS> row;
+    row.first(q, kc, vc, nq, nkv, HD, max_seq, h, t, (int)threadIdx.x & (kAttnThreads - 1));
+    const int p0 = *pos0;
+    if (min(p0 + T, (int)max_seq) <= kFaRowKeys) {
+      if (2 * wg >= units) return;
+      float *const s_acc = reinterpret_cast<float *>(&s_kv[0][0][0]) + half * kUnit;
+      float *const s_p = s_acc + kAcc;
+      row.finish(min(p0 + t + 1, (int)max_seq), scaling, out + ((size_t)t * nq + h) * HD, s_p, kFaRowKeys,
+                 s_p + ROWS * kFaRowKeys, s_acc);
+      return;
+    }
+  }
 
   const int tid = threadIdx.x & (kFaHalf - 1);
   const int lane = tid & (kWave - 1);
@@ -575,7 +647,7 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
 
   // The first split's first pair of tiles is loaded with q and the position.
   const int split = (int)blockIdx.y;
-  if (split == 0) load(kgrp * kFaKeys);
+  if (ROWS == 0 && split == 0) load(kgrp * kFaKeys);
   const int p0 = *pos0;
   const int limit = min(p0 + t + 1, cap);  // keys 0 .. limit - 1 of this lane's row
   const int nkeys = min(p0 + min(row0 + kFaRows - 1, rows - 1) / grp + 1, cap);  // of the last row
@@ -586,20 +658,25 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
       for (int d = hh * 4; d < HD; d += 8) *reinterpret_cast<uint2 *>(orow + d) = make_uint2(0u, 0u);
     return;  // uniform over the workgroup
   }
-  // Pairs [it0, it1) are this split's.
+  // Pairs [it0, it1) are this split's: two at least with one or two pairs in all (32 tokens
+  // behind 100 keys: 13.8 us in two splits, 12.3 in one) and from eight (40 behind 1000: 20.8
+  // and 19.6), as a split's partial output costs about what a pair does.
   const int npair = (nkeys + 2 * kFaKeys - 1) / (2 * kFaKeys);
-  const int per = (npair + (int)gridDim.y - 1) / (int)gridDim.y;
+  const int per = max(npair <= 2 || npair >= 8 ? 2 : 1, (npair + splits - 1) / splits);
   const int nact = (npair + per - 1) / per;  // splits with work
   if (split >= nact) return;                 // uniform over the workgroup
   const int it0 = split * per, it1 = min(it0 + per, npair);
   const int kend = min(nkeys, it1 * 2 * kFaKeys);
-  if (split > 0) load((2 * it0 + kgrp) * kFaKeys);
+  if (ROWS > 0 || split > 0) load((2 * it0 + kgrp) * kFaKeys);
   bool nonfinite = false;
+  if (threadIdx.x == 0) s_nonfinite = 0;  // (the first pair's barrier follows)
+  const int nfull = min(max(max(first, 0) / (2 * kFaKeys), it0), it1);
+  const bool lone = it1 - it0 == 1 && nfull == it0;
   // One pair of tiles.  EDGE: some row of the workgroup stops inside the pair.
   auto pair = [&](int it, auto edge_c) __attribute__((always_inline)) {
     constexpr bool kEdge = decltype(edge_c)::value;
-    const int k0 = (2 * it + kgrp) * kFaKeys;
-    uint8_t *const buf = s_kv[(it - it0) & 1][kgrp];
+    int k0 = (2 * it + kgrp) * kFaKeys;
+    uint8_t *buf = s_kv[(it - it0) & 1][kgrp];
     uint32_t kx = krx, vx = vrx;
     asm volatile("" : "+v"(kx), "+v"(vx));
     if constexpr (kEdge) {
@@ -618,71 +695,86 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
     stage(buf);
     __syncthreads();
     if (it + 1 < it1) load(k0 + 2 * kFaKeys);
-
-    f32x16 sc[2];
+    auto tile = [&]() __attribute__((always_inline)) {
+      f32x16 sc[2];
 #pragma unroll
-    for (int st = 0; st < 2; ++st)
+      for (int st = 0; st < 2; ++st)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) sc[st][v] = 0.0f;
+        for (int v = 0; v < 16; ++v) sc[st][v] = 0.0f;
 #pragma unroll
-    for (int s = 0; s < HD / 16; ++s) {
+      for (int s = 0; s < HD / 16; ++s) {
 #pragma unroll
-      for (int st = 0; st < 2; ++st) {
-        const u32x4 a = *reinterpret_cast<const u32x4 *>(buf + krd + (kx ^ (32 * s)) + 32 * st * (2 * HD));
-        sc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa_op(a), fa_op(qf[s]), sc[st], 0, 0, 0);
+        for (int st = 0; st < 2; ++st) {
+          const u32x4 a = *reinterpret_cast<const u32x4 *>(buf + krd + (kx ^ (32 * s)) + 32 * st * (2 * HD));
+          sc[st] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa_op(a), fa_op(qf[s]), sc[st], 0, 0, 0);
+        }
+      }
+      float mx = -INFINITY;
+#pragma unroll
+      for (int st = 0; st < 2; ++st)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          float x = bf16r(bf16r(sc[st][v]) * scaling);
+          if constexpr (kEdge) x = k0 + 32 * st + 8 * (v >> 2) + 4 * hh + (v & 3) < limit ? x : -INFINITY;
+          sc[st][v] = x;
+          mx = fmaxf(mx, x);
+        }
+      mx = op_xor32<true>(mx);
+      const float mn = fmaxf(m, mx);
+      // Before a row's first key (none of its keys so far above -inf): any finite reference.
+      const float mref = mn == -INFINITY ? 0.0f : mn;
+      if (__any(mn > m)) {
+        const float alpha = __builtin_amdgcn_exp2f((m - mref) * kLog2e);
+        l *= alpha;
+#pragma unroll
+        for (int dt = 0; dt < kDT; ++dt)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[dt][v] *= alpha;
+        m = mn;
+      }
+      u32x4 pf[4];
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int v = 8 * (s & 1) + 2 * j;
+          // (The difference first: mref * kLog2e alone overflows from 2.36e38.)
+          const float e0 = __builtin_amdgcn_exp2f((sc[s >> 1][v] - mref) * kLog2e);
+          const float e1 = __builtin_amdgcn_exp2f((sc[s >> 1][v + 1] - mref) * kLog2e);
+          l += e0 + e1;
+          pf[s][j] = pack_bf16x2(e0, e1);
+        }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int dt = 0; dt < kDT; ++dt) {
+          const u32x4 a = *reinterpret_cast<const u32x4 *>(
+              buf + vrd + (vx ^ (16 * ((2 * s) ^ ((2 * dt) & 7)))) + 32 * dt * (2 * kFaKeys));
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa_op(a), fa_op(pf[s]), acc[dt], 0, 0, 0);
+        }
+    };
+    if constexpr (!kEdge) {
+      tile();
+    } else {
+      // A workgroup with this one pair: group 0 takes both tiles (nothing to join), else each
+      // group its own.
+      k0 = (2 * it + (lone ? 0 : kgrp)) * kFaKeys;
+      buf = s_kv[(it - it0) & 1][lone ? 0 : kgrp];
+#pragma unroll 1
+      for (int n = lone ? 2 - 2 * kgrp : 1; n > 0 && k0 < kend; --n) {
+        tile();
+        k0 += kFaKeys;
+        buf += kKPlane + kVPlane;
       }
     }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int st = 0; st < 2; ++st)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        float x = bf16r(bf16r(sc[st][v]) * scaling);
-        if constexpr (kEdge) x = k0 + 32 * st + 8 * (v >> 2) + 4 * hh + (v & 3) < limit ? x : -INFINITY;
-        sc[st][v] = x;
-        mx = fmaxf(mx, x);
-      }
-    mx = op_xor32<true>(mx);
-    const float mn = fmaxf(m, mx);
-    // Before a row's first key (none of its keys so far above -inf): any finite reference.
-    const float mref = mn == -INFINITY ? 0.0f : mn;
-    if (__any(mn > m)) {
-      const float alpha = __builtin_amdgcn_exp2f((m - mref) * kLog2e);
-      l *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < kDT; ++dt)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[dt][v] *= alpha;
-      m = mn;
-    }
-    u32x4 pf[4];
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int v = 8 * (s & 1) + 2 * j;
-        // (The difference first: mref * kLog2e alone overflows from 2.36e38.)
-        const float e0 = __builtin_amdgcn_exp2f((sc[s >> 1][v] - mref) * kLog2e);
-        const float e1 = __builtin_amdgcn_exp2f((sc[s >> 1][v + 1] - mref) * kLog2e);
-        l += e0 + e1;
-        pf[s][j] = pack_bf16x2(e0, e1);
-      }
-#pragma unroll
-    for (int s = 0; s < 4; ++s)
-#pragma unroll
-      for (int dt = 0; dt < kDT; ++dt) {
-        const u32x4 a = *reinterpret_cast<const u32x4 *>(
-            buf + vrd + (vx ^ (16 * ((2 * s) ^ ((2 * dt) & 7)))) + 32 * dt * (2 * kFaKeys));
-        acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa_op(a), fa_op(pf[s]), acc[dt], 0, 0, 0);
-      }
   };
   // Pairs that every row sees whole, then the (at most two or so) where rows stop: apart, so
   // that the long loop has no masks and keeps all its values in registers.
-  const int nfull = min(max(max(first, 0) / (2 * kFaKeys), it0), it1);
   for (int it = it0; it < nfull; ++it) pair(it, std::false_type{});
   for (int it = nfull; it < it1; ++it) pair(it, std::true_type{});
-  // (Also the barrier before the planes are reused.)
-  if (__syncthreads_or(nonfinite ? 1 : 0)) {
+  if (nonfinite) s_nonfinite = 1;
+  __syncthreads();  // (also the barrier before the planes are reused)
+  if (s_nonfinite != 0) {
     // Row by row, a wave per row and a key per lane, so that each row reads the V rows that
     // it sees and no others.
     fa_rows_scalar<HD>(q, kbase, vbase, row0, min(row0 + kFaRows, rows), it0 * 2 * kFaKeys, kend, p0, cap,
@@ -701,33 +793,41 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
   } else {
     l = op_xor32<false>(l);
   }
-  // Key group 1's maxima, sums and output join group 0's through LDS: word v of a lane at
-  // [row group][v][lane].
-  float *const s_o = reinterpret_cast<float *>(&s_kv[0][0][0]);
-  static_assert(4 * (16 * kDT + 2) * kWave * 4 <= (int)sizeof(s_kv), "partial outputs fit the planes");
-  float *const mine = s_o + wave * (16 * kDT + 2) * kWave + lane;
-  if (kgrp == 1) {
+  // Key group 1's maxima, sums and output join group 0's through LDS, four words of a lane at
+  // [row group][quad][lane].
+  if (!lone) {
+    float4 *const s_o = reinterpret_cast<float4 *>(&s_kv[0][0][0]);
+    static_assert(4 * (4 * kDT + 1) * kWave * 16 <= (int)sizeof(s_kv), "partial outputs fit the planes");
+    float4 *const mine = s_o + wave * (4 * kDT + 1) * kWave + lane;
+    if (kgrp == 1) {
 #pragma unroll
-    for (int dt = 0; dt < kDT; ++dt)
+      for (int dt = 0; dt < kDT; ++dt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) mine[(16 * dt + v) * kWave] = acc[dt][v];
-    mine[16 * kDT * kWave] = m;
-    mine[(16 * kDT + 1) * kWave] = l;
-  }
-  __syncthreads();
-  // From here on key group 1's waves only keep the barriers.
-  if (kgrp == 0) {
-    const float m1 = mine[16 * kDT * kWave], l1 = mine[(16 * kDT + 1) * kWave];
-    const float mn = fmaxf(m, m1);
-    const float mref = mn == -INFINITY ? 0.0f : mn;
-    const float a0 = __builtin_amdgcn_exp2f((m - mref) * kLog2e);
-    const float a1 = __builtin_amdgcn_exp2f((m1 - mref) * kLog2e);
-    m = mn;
-    l = l * a0 + l1 * a1;
+        for (int v = 0; v < 16; v += 4)
+          mine[(4 * dt + v / 4) * kWave] = make_float4(acc[dt][v], acc[dt][v + 1], acc[dt][v + 2], acc[dt][v + 3]);
+      mine[4 * kDT * kWave] = make_float4(m, l, 0.0f, 0.0f);
+    }
+    __syncthreads();
+    // From here on key group 1's waves only keep the barriers.
+    if (kgrp == 0) {
+      const float4 ml = mine[4 * kDT * kWave];
+      const float mn = fmaxf(m, ml.x);
+      const float mref = mn == -INFINITY ? 0.0f : mn;
+      const float a0 = __builtin_amdgcn_exp2f((m - mref) * kLog2e);
+      const float a1 = __builtin_amdgcn_exp2f((ml.x - mref) * kLog2e);
+      m = mn;
+      l = l * a0 + ml.y * a1;
 #pragma unroll
-    for (int dt = 0; dt < kDT; ++dt)
+      for (int dt = 0; dt < kDT; ++dt)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[dt][v] = acc[dt][v] * a0 + mine[(16 * dt + v) * kWave] * a1;
+        for (int v = 0; v < 16; v += 4) {
+          const float4 o = mine[(4 * dt + v / 4) * kWave];
+          acc[dt][v] = acc[dt][v] * a0 + o.x * a1;
+          acc[dt][v + 1] = acc[dt][v + 1] * a0 + o.y * a1;
+          acc[dt][v + 2] = acc[dt][v + 2] * a0 + o.z * a1;
+          acc[dt][v + 3] = acc[dt][v + 3] * a0 + o.w * a1;
+        }
+    }
   }
   if (nact > 1) {
     // Partial results to the workspace, word w of a lane at [w][lane] of its wave's block;
@@ -735,7 +835,7 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
     // (its own too is read back), and writes the rows.
     constexpr int kWords = (16 * kDT + 2) * kWave;
     const int unit = (int)blockIdx.x;
-    float *const pu = part + ((size_t)unit * gridDim.y * 4 + wave) * kWords + lane;
+    float *const pu = part + ((size_t)unit * splits * 4 + wave) * kWords + lane;
     const bool live = kgrp == 0 && row0 + wave * 32 < rows;  // waves without rows have nothing
     if (live) {
       float *const pw = pu + (size_t)split * 4 * kWords;
@@ -793,16 +893,19 @@ constexpr int64_t kAttnUnitsMax = kAttnCounterBytes / 4;
 // Launch plan of a call: which kernel, its splits of the keys, and the workspace it needs.
 struct AttnPlan {
   bool matrix;     // prefill_attention_kernel
+  int rows;        // its instance that takes short contexts by rows (heads a unit; 0: none)
   int64_t units;   // workgroups per split
   int splits;
   int64_t bytes;   // workspace (0: none)
 };
 
 AttnPlan attn_plan(int64_t T, int32_t nq, int32_t nkv, int32_t hd, int64_t max_seq, bool ws) {
-  AttnPlan p{false, nq, 1, 0};
+  AttnPlan p{false, 0, nq, 1, 0};
   const int64_t rows = T * (nq / nkv);
   if (T > kFewTokens && (hd == 64 || hd == 128)) {
     p.matrix = true;
+    const int64_t fit = 2 * (int64_t)device_cu_count();  // units at a time
+    p.rows = nq * T <= fit ? 1 : nq / nkv % 2 == 0 && nq / 2 * T <= fit ? 2 : 0;
     p.units = (rows + kFaRows - 1) / kFaRows * nkv;
     // Row tiles alone do not fill the chip: share a tile's keys, down to two pairs of key
     // tiles per split.
@@ -885,9 +988,18 @@ extern "C" int moe_attention_ws_bf16(const void *q, const void *k_cache, const v
   const bool matrix = p.matrix && (uintptr_t)out % 8 == 0 &&
                       T * (int64_t)(n_q_heads / n_kv_heads) <= 0x7fffffff - moe::kFaRows && p.units <= 0x7fffffff;
   if (matrix) {
-    auto kern = head_dim == 64 ? moe::prefill_attention_kernel<64> : moe::prefill_attention_kernel<128>;
-    hipLaunchKernelGGL(kern, dim3((unsigned)p.units, (unsigned)p.splits), dim3(moe::kFaThreads), 0, s, qp,
-                       kp, vp, (int)T, n_q_heads, n_kv_heads, pp, max_seq, scaling, op, count, part);
+    auto kern = head_dim == 64 ? (p.rows == 0   ? moe::prefill_attention_kernel<64, 0>
+                                  : p.rows == 1 ? moe::prefill_attention_kernel<64, 1>
+                                                : moe::prefill_attention_kernel<64, 2>)
+                               : (p.rows == 0   ? moe::prefill_attention_kernel<128, 0>
+                                  : p.rows == 1 ? moe::prefill_attention_kernel<128, 1>
+                                                : moe::prefill_attention_kernel<128, 2>);
+    // The row instances: a workgroup for every two units at least.
+    const int64_t row_wgs = p.rows > 0 ? (n_q_heads / p.rows * T + 1) / 2 : 0;
+    const int64_t row_y = (row_wgs + p.units - 1) / p.units;
+    const unsigned y = (unsigned)(row_y > p.splits ? row_y : p.splits);
+    hipLaunchKernelGGL(kern, dim3((unsigned)p.units, y), dim3(moe::kFaThreads), 0, s, qp, kp, vp, (int)T,
+                       n_q_heads, n_kv_heads, pp, max_seq, scaling, op, count, part, p.splits);
   } else if (!p.matrix && p.splits > 1) {
     hipLaunchKernelGGL(moe::few_attention_kernel, dim3((unsigned)n_q_heads, (unsigned)p.splits, (unsigned)T),
                        dim3(moe::kAttnThreads), 0, s, qp, kp, vp, n_q_heads, n_kv_heads, head_dim, pp,

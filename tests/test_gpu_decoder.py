@@ -150,14 +150,19 @@ def _attend_ref(q, k, v, p0, scaling=None):
 
 
 # Above 8 tokens the matrix form: row tiles of 128 (token, head of the group) rows, key tiles
-# of 64 keys, taken in pairs.  Up to 8 tokens a row's keys are shared between workgroups above
-# 384 of them.
+# of 64 keys, taken in pairs (a lone pair by one wave group); up to 384 keys its row instances
+# where the units, 1 or 2 heads of a token, are 512 or fewer.  Up to 8 tokens a row's keys are
+# shared between workgroups above 384 of them.
 @pytest.mark.parametrize("T,p0,max_seq,nq,nkv,hd", [
     (17, 0, 64, 4, 4, 128), (18, 46, 64, 8, 2, 64), (2, 0, 64, 4, 4, 128), (9, 50, 64, 8, 2, 64), (8, 380, 400, 8, 2, 64), (33, 95, 128, 32, 8, 128), (32, 128, 256, 4, 1, 128),
     (129, 0, 256, 2, 2, 64), (65, 127, 200, 6, 2, 128), (17, 700, 1024, 8, 8, 64),
     (5, 2500, 4096, 32, 8, 128), (40, 1000, 2048, 7, 1, 128),
     (1, 383, 4096, 32, 8, 128), (1, 384, 4096, 32, 8, 128), (1, 640, 1000, 6, 3, 64),
-    (1, 8191, 8192, 8, 8, 256), (1, 2900, 4096, 8, 8, 128)])
+    (1, 8191, 8192, 8, 8, 256), (1, 2900, 4096, 8, 8, 128),
+    (129, 0, 256, 16, 2, 64), (65, 127, 200, 24, 4, 128), (66, 64, 130, 16, 16, 128),
+    (100, 0, 128, 16, 4, 128), (60, 0, 64, 32, 8, 64), (60, 68, 128, 32, 8, 128),
+    (16, 368, 400, 32, 8, 128), (16, 369, 400, 32, 8, 128), (9, 5, 64, 7, 7, 64),
+    (30, 300, 400, 32, 4, 128), (17, 3, 64, 34, 17, 64)])
 def test_attention_forms(cuda_device, T, p0, max_seq, nq, nkv, hd):
     """Matrix form and shared keys: against the module's arithmetic, with cache rows past the
     last key NaN; the workspace's counters return to zero, a second call repeats the bits."""
@@ -180,12 +185,13 @@ def test_attention_forms(cuda_device, T, p0, max_seq, nq, nkv, hd):
     assert torch.equal(_attend(qd, kd, vd, p0, ws), got)
 
 
-@pytest.mark.parametrize("T,p0,hd", [(40, 70, 128), (130, 0, 64), (20, 1500, 128), (6, 1500, 128)])
-def test_attention_nonfinite_values(cuda_device, T, p0, hd):
+@pytest.mark.parametrize("T,p0,hd,nq", [(40, 70, 128, 8), (130, 0, 64, 8), (20, 1500, 128, 8), (6, 1500, 128, 8),
+                                        (60, 40, 128, 32), (50, 0, 64, 32), (40, 100, 128, 32)])
+def test_attention_nonfinite_values(cuda_device, T, p0, hd, nq):
     """An infinity or NaN in a V row reaches the queries that see the row and no others."""
     from moeinfra_amd import _lib
 
-    nq, nkv, max_seq, S = 8, 2, 2048, p0 + T
+    nkv, max_seq, S = 2, 2048, p0 + T
     q, k, v = _bf16((T, nq, hd), 15), _bf16((nkv, S, hd), 16), _bf16((nkv, S, hd), 17)
     clean = v.clone()
     bad = p0 + T // 2
@@ -302,6 +308,27 @@ def test_attention_splits_join_in_order(cuda_device, hd):
         got = _attend(q, k, v, p0, ws)
         # one bf16 rounding (a lost split is 3.4 % off)
         assert torch.allclose(got.float(), want, rtol=2.0 ** -8, atol=0.0)
+
+
+@pytest.mark.parametrize("T,p0,nq,nkv,hd", [(9, 0, 32, 8, 128), (16, 368, 32, 8, 128), (13, 40, 7, 7, 64),
+                                            (17, 0, 32, 8, 128), (32, 352, 32, 8, 128), (17, 100, 34, 17, 64)])
+def test_attention_short_context_by_rows(cuda_device, T, p0, nq, nkv, hd):
+    """A few dozen tokens with up to 384 keys run row by row: each token's outputs have the bits
+    of a call of that token alone (pairs of key tiles on the matrix cores took these prompts
+    twice as long and round the probabilities before the division)."""
+    from moeinfra_amd import _lib
+
+    max_seq, S = 400, p0 + T
+    q, k, v = _bf16((T, nq, hd), 55), _bf16((nkv, S, hd), 56), _bf16((nkv, S, hd), 57)
+    kc = torch.full((nkv, max_seq, hd), float("nan"), dtype=torch.bfloat16)
+    vc = kc.clone()
+    kc[:, :S], vc[:, :S] = k, v
+    qd, kd, vd = q.to(cuda_device), kc.to(cuda_device), vc.to(cuda_device)
+    n = _lib.lib().moe_attention_workspace_bytes(T, nq, nkv, hd, max_seq)
+    ws = torch.zeros((max(n, 16),), dtype=torch.uint8, device=cuda_device)
+    want = torch.cat([_attend(qd[t:t + 1], kd, vd, p0 + t, None) for t in range(T)])
+    for w in (None, ws):
+        np.testing.assert_array_equal(bits(_attend(qd, kd, vd, p0, w)), bits(want))
 
 
 @pytest.mark.parametrize("T,N,K", [(1, 6144, 4096), (1, 4096, 4096), (1, 1000, 512), (4, 515, 1024)])
