@@ -902,9 +902,12 @@ struct AttnPlan {
 AttnPlan attn_plan(int64_t T, int32_t nq, int32_t nkv, int32_t hd, int64_t max_seq, bool ws) {
   AttnPlan p{false, 0, nq, 1, 0};
   const int64_t rows = T * (nq / nkv);
-  if (T > kFewTokens && (hd == 64 || hd == 128)) {
+  const int64_t fit = 2 * (int64_t)device_cu_count();  // (head, token) units at a time
+  // Without a workspace no keys are shared, and a row tile's one workgroup has a longer chain
+  // than the rows' own while those run all at once (9 tokens behind 1000 keys: 26 us, 22 with a
+  // workgroup per row; 8 heads of 64, 16 tokens: 20 and 11; 64 tokens of 32 heads: 30 and 75).
+  if (T > kFewTokens && (hd == 64 || hd == 128) && (ws || nq * T > fit)) {
     p.matrix = true;
-    const int64_t fit = 2 * (int64_t)device_cu_count();  // units at a time
     p.rows = nq * T <= fit ? 1 : nq / nkv % 2 == 0 && nq / 2 * T <= fit ? 2 : 0;
     p.units = (rows + kFaRows - 1) / kFaRows * nkv;
     // Row tiles alone do not fill the chip: share a tile's keys, down to two pairs of key

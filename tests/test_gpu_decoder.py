@@ -331,6 +331,18 @@ def test_attention_short_context_by_rows(cuda_device, T, p0, nq, nkv, hd):
         np.testing.assert_array_equal(bits(_attend(qd, kd, vd, p0, w)), bits(want))
 
 
+@pytest.mark.parametrize("T,p0,nq,nkv,hd", [(9, 1000, 32, 8, 128), (16, 500, 8, 8, 64), (60, 700, 8, 1, 128)])
+def test_attention_without_workspace(cuda_device, T, p0, nq, nkv, hd):
+    """Without a workspace to share keys through, rows that the device holds all at once run one
+    workgroup each, at any context length: the bits of one-token calls."""
+    max_seq, S = 1100, p0 + T
+    q, k, v = _bf16((T, nq, hd), 65), _bf16((nkv, max_seq, hd), 66), _bf16((nkv, max_seq, hd), 67)
+    qd, kd, vd = q.to(cuda_device), k.to(cuda_device), v.to(cuda_device)
+    want = torch.cat([_attend(qd[t:t + 1], kd, vd, p0 + t, None) for t in range(T)])
+    np.testing.assert_array_equal(bits(_attend(qd, kd, vd, p0, None)), bits(want))
+    assert rel_l2(want.cpu(), _attend_ref(q, k[:, :S], v[:, :S], p0)) < 4e-3
+
+
 @pytest.mark.parametrize("T,N,K", [(1, 6144, 4096), (1, 4096, 4096), (1, 1000, 512), (4, 515, 1024)])
 def test_gemv(cuda_device, T, N, K):
     from moeinfra_amd import _lib
