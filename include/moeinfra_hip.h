@@ -187,10 +187,13 @@ int moe_expert_swiglu_nf4(const moe_nf4_expert_t *expert, const void *x_bf16, in
  * receive the routing.  workspace >= moe_layer_workspace_bytes(T, k, E, H, F), 256-byte
  * aligned. */
 int64_t moe_layer_workspace_bytes(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F);
-/* Number of fp32 ypart planes (K splits of the down projection) the layer and the expert
- * FFN use by default for this shape: what moe_expert_ffn_nf4 / moe_expert_down_nf4 callers
- * pass as nsplit to run the layer's kernels (sizing helper, like the workspace query; the
- * reference has no K splits).  -1 for invalid sizes. */
+/* Number of fp32 ypart planes (K splits of the down projection) by default for this shape:
+ * what callers of the separate calls, moe_expert_ffn_nf4 / moe_expert_down_nf4, pass as nsplit
+ * (sizing helper, like the workspace query; the reference has no K splits).  The whole calls,
+ * moe_layer_forward_nf4 and moe_expert_swiglu_nf4, use as many, except where their down
+ * projection is cut by the routed counts (batches of 32 and more rows per expert: ranges, with
+ * planes of their own): there the two agree up to the order of fp32 sums.  -1 for invalid
+ * sizes. */
 int32_t moe_layer_down_splits(int64_t T, int32_t k, int32_t E, int32_t H, int32_t F);
 int moe_layer_forward_nf4(const moe_nf4_expert_t *experts, int32_t E, const void *gate_bf16,
                           const void *bias_f32, const void *x_bf16, int64_t T, int32_t H,
@@ -266,16 +269,19 @@ int moe_rope_kv_bf16(const void *qkv, int64_t T, int32_t n_q_heads, int32_t n_kv
 
 /* Grouped-query causal attention of q [T, n_q, head_dim] (query t at position *pos0 + t)
  * against the caches: bf16(bf16(q.k) * scaling) scores, fp32 softmax rounded to bf16,
- * fp32-accumulated sum of the probabilities times v; out [T, n_q * head_dim]. */
+ * fp32-accumulated sum of the probabilities times v; out [T, n_q * head_dim].  More than 8
+ * tokens of head dim 64 or 128, with more than two rows (query heads of a token) per CU: matrix
+ * products, the probabilities rounded before the division by their sum. */
 int moe_attention_bf16(const void *q, const void *k_cache, const void *v_cache, int64_t T,
                        int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
                        const void *pos0_i32, int64_t max_seq, float scaling, void *out,
                        void *stream);
 
-/* The same with a workspace, so that several
- * workgroups can share a row's keys when the rows alone do not fill the device: one token
- * behind more than 512 keys, few tokens behind a long context.  Their probabilities are
- * rounded before the division by the sum (several tokens) or not at all (one token).
+/* The same with a workspace, so that several workgroups can share a row's keys when the rows
+ * alone do not fill the device.  Up to 8 tokens share the keys of rows that see more than 384
+ * and round no probability; more tokens (head dim 64 or 128) run as matrix products, rounded
+ * before the division, except a few dozen with up to 384 keys, whose rows have the bits of
+ * one-token calls.  The partial results of shared keys add up in a fixed order.
  * moe_attention_workspace_bytes: what any call of 1 .. T tokens needs.  The workspace is
  * 16-byte aligned and its first 4096 bytes are zero before the first call (every call leaves
  * them zero); calls that share it must be ordered (one stream).  Null: moe_attention_bf16. */

@@ -851,7 +851,12 @@ expert_gemm_kernel(const ExpertTable tab, const uint16_t *__restrict__ act, uint
 
 // Kernel shape of a launch (waves, token tiles per item, fragments per wave, ring depth):
 // 256-token items (W = 4, MT = 8) from 512 routed rows per active expert on average, else
-// 128-token items with two waves per SIMD (W = 8, MT = 4).
+// 128-token items with two waves per SIMD (W = 8, MT = 4).  Both sides of the line, in 128- and
+// 256-token items: hidden 4096, 8 experts, 425 / 500 / 575 rows each 1413 / 1594 / 1850 and 1290
+// / 1536 / 1729 us; hidden 3072, 450 / 525 rows 657 / 766 and 697 / 779; 16 experts, hidden 2048,
+// 450 / 525 rows 784 / 946 and 755 / 958 (skewed 773 / 895 and 835 / 911); one expert of 460 /
+// 560 rows 209 / 323 and 193 / 303.  With 4096 and for one expert the line could be lower, for
+// the other shapes not.
 struct GemmShape {
   int waves, mt, nf, bd;
   int64_t tokens() const { return 32 * mt; }
