@@ -78,6 +78,9 @@ constexpr int kQuantThreads = 256;
 // (4.1 TB/s; 48 us while every thread built eight table entries and no load ran ahead).  The
 // entry {midpoint, count below the bin} has 32 replicas
 // (conflict-free ds_read_b64).  A codebook with two midpoints in a bin compares with all 15.
+// So do weights with at most one chunk a wave (TABLE false): every workgroup builds the table for
+// itself, half a microsecond that one chunk does not earn back (512 / 1 M / 4 M values: 3.2 / 4.0
+// / 6.4 us with the table, 2.6 / 3.2 / 6.2 without; 5 M, two chunks: 6.4 and 7.2).
 constexpr int kQuant64Chunk = 512;
 constexpr int kQuantBins = 64;
 constexpr int kQuantReps = 32;
@@ -89,7 +92,7 @@ __device__ __forceinline__ uint32_t quant_bin(float y) {
 }
 
 template <bool BINS>
-__device__ __forceinline__ uint32_t quant8(const u32x4 raw, float r, const float *mid, const float2 *bins,
+__device__ __forceinline__ uint32_t quant8(const u32x4 raw, float r, const float (&mid)[15], const float2 *bins,
                                            uint32_t rep) {
   uint32_t out = 0;
 #pragma unroll
@@ -100,6 +103,7 @@ __device__ __forceinline__ uint32_t quant8(const u32x4 raw, float r, const float
       const float2 e = bins[quant_bin(y) * kQuantReps + rep];
       q = __builtin_bit_cast(uint32_t, e.y) + (y > e.x ? 1u : 0u);
     } else {
+#pragma unroll
       for (int m = 0; m < 15; ++m) q += y > mid[m] ? 1u : 0u;
     }
     // value 2j in the high nibble of byte j
@@ -110,25 +114,34 @@ __device__ __forceinline__ uint32_t quant8(const u32x4 raw, float r, const float
 
 template <bool BINS>
 __device__ __forceinline__ void quant64_chunks(const uint16_t *w, int64_t nchunk, uint8_t *packed, float *absmax,
-                                               const float *mid, const float2 *bins) {
+                                               const float *s_mid, const float2 *bins) {
+  float mid[15];
+#pragma unroll
+  for (int m = 0; m < 15; ++m) mid[m] = BINS ? 0.0f : s_mid[m];
   const int lane = threadIdx.x & (kWave - 1);
   const uint32_t rep = threadIdx.x & (kQuantReps - 1);
   const int64_t waves = (int64_t)gridDim.x * (kQuantThreads / kWave);
   const int64_t c0 = (int64_t)blockIdx.x * (kQuantThreads / kWave) + (threadIdx.x >> 6);
-  // Two chunks per step, the next step's loads in flight under this one's arithmetic (past
-  // the end: the last chunk again, unused).
   auto load = [&](int64_t c) {
     const uint4 v = ld_stream16(w + (c < nchunk ? c : nchunk - 1) * kQuant64Chunk + 8 * lane);
     return u32x4{v.x, v.y, v.z, v.w};
   };
-  u32x4 next[2] = {load(c0), load(c0 + waves)};
-  for (int64_t c = c0; c < nchunk; c += 2 * waves) {
-    const u32x4 raw[2] = {next[0], next[1]};
-    next[0] = load(c + 2 * waves);
-    next[1] = load(c + 3 * waves);
-    float amax[2] = {0.0f, 0.0f};
+  // With the table two chunks per step, the next step's loads in flight under this one's
+  // arithmetic (past the end: the last chunk again, unused).
+  constexpr int kStep = BINS ? 2 : 1;
+  u32x4 next[kStep];
+  if constexpr (BINS)
+    for (int u = 0; u < kStep; ++u) next[u] = load(c0 + u * waves);
+  for (int64_t c = c0; c < nchunk; c += kStep * waves) {
+    u32x4 raw[kStep];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < kStep; ++u) {
+      raw[u] = BINS ? next[u] : load(c);
+      if constexpr (BINS) next[u] = load(c + (u + kStep) * waves);
+    }
+    float amax[kStep] = {};
+#pragma unroll
+    for (int u = 0; u < kStep; ++u)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         amax[u] = fmaxf(amax[u], fabsf(bf16lo_to_f32(raw[u][i])));
@@ -136,8 +149,8 @@ __device__ __forceinline__ void quant64_chunks(const uint16_t *w, int64_t nchunk
       }
     lane_groups_reduce<true>(amax, 8);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
-      if (u == 1 && c + waves >= nchunk) break;
+    for (int u = 0; u < kStep; ++u) {
+      if (u > 0 && c + u * waves >= nchunk) break;
       const int64_t v0 = (c + u * waves) * kQuant64Chunk + 8 * lane;
       if ((lane & 7) == 0) absmax[v0 / 64] = amax[u];
       const float r = amax[u] > 0.0f ? 1.0f / amax[u] : 0.0f;
@@ -146,15 +159,20 @@ __device__ __forceinline__ void quant64_chunks(const uint16_t *w, int64_t nchunk
   }
 }
 
+template <bool TABLE>
 __global__ void __launch_bounds__(kQuantThreads)
 nf4_quantize64_kernel(const uint16_t *__restrict__ w, int64_t nchunk,
                       const float *__restrict__ code, uint8_t *__restrict__ packed,
                       float *__restrict__ absmax, float *__restrict__ code_out) {
   __shared__ float s_mid[15];
-  __shared__ float2 s_bins[kQuantBins * kQuantReps];
+  __shared__ float2 s_bins[TABLE ? kQuantBins * kQuantReps : 1];
   if (threadIdx.x < 15) s_mid[threadIdx.x] = (code[threadIdx.x] + code[threadIdx.x + 1]) * 0.5f;
   if (code_out != nullptr && blockIdx.x == 0 && threadIdx.x < 16) code_out[threadIdx.x] = code[threadIdx.x];
   __syncthreads();
+  if constexpr (!TABLE) {
+    quant64_chunks<false>(w, nchunk, packed, absmax, s_mid, s_bins);
+    return;
+  }
   // One thread per bin, then the replicas.
   int crowded = 0;
   if (threadIdx.x < kQuantBins) {
@@ -297,7 +315,9 @@ extern "C" int moe_nf4_quantize_state_bf16(const void *w_bf16, int64_t numel, in
     int64_t blocks = (nchunk + (moe::kQuantThreads / moe::kWave) - 1) / (moe::kQuantThreads / moe::kWave);
     const int64_t cap = (int64_t)moe::device_cu_count() * 8;
     blocks = blocks > cap ? cap : blocks;
-    hipLaunchKernelGGL(moe::nf4_quantize64_kernel, dim3((unsigned)blocks), dim3(moe::kQuantThreads),
+    const bool table = nchunk > blocks * (moe::kQuantThreads / moe::kWave);  // more than a chunk a wave
+    auto kern = table ? moe::nf4_quantize64_kernel<true> : moe::nf4_quantize64_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(moe::kQuantThreads),
                        0, (hipStream_t)stream, (const uint16_t *)w_bf16, nchunk,
                        (const float *)code16, (uint8_t *)packed_out, (float *)absmax_out,
                        (float *)code_out);
