@@ -84,31 +84,35 @@ struct AttnRow {
     for (int u = 0; u < kAttnRowsInFlight; ++u)
       dst[u] = *reinterpret_cast<const uint4 *>(base + (size_t)min(j0 + u * rpp + rr, last) * hd);
   }
-  // Heads h .. h + NH - 1 of one KV head.
-  __device__ __forceinline__ void first(const uint16_t *q, const uint16_t *kc, const uint16_t *vc, int nq, int nkv,
-                                        int hd_, int64_t max_seq, int h, int t, int tid_) {
+  __device__ __forceinline__ void place(const uint16_t *kc, const uint16_t *vc, int kvh, int hd_,
+                                        int64_t max_seq, int tid_) {
     tid = tid_;
     hd = hd_;
     lpr = hd >> 3;               // lanes per row: a power of two <= 32
     rpp = kAttnThreads / lpr;    // rows per load instruction
     sub = tid & (lpr - 1);
     rr = tid / lpr;
+    kbase = kc + (size_t)kvh * max_seq * hd + sub * 8;
+    vbase = vc + (size_t)kvh * max_seq * hd + sub * 8;
+  }
+  // q (heads h .. h + NH - 1 of row t, of the KV head) and the first pass's rows, up to row `last` of the keys at kbase / vbase.
+  __device__ __forceinline__ void first(const uint16_t *q, int nq, int h, int t, int last) {
 #pragma unroll
     for (int n = 0; n < NH; ++n)
       unpack8(*reinterpret_cast<const uint4 *>(q + ((size_t)t * nq + h + n) * hd + sub * 8), qf[n]);
-    const int kvh = h / (nq / nkv);
-    kbase = kc + (size_t)kvh * max_seq * hd + sub * 8;
-    vbase = vc + (size_t)kvh * max_seq * hd + sub * 8;
-    load(kv, kbase, 0, (int)max_seq - 1);
-    load(vv, vbase, 0, (int)max_seq - 1);
+    load(kv, kbase, 0, last);
+    load(vv, vbase, 0, last);
   }
-  // The NH output rows at `orow` over nkeys keys.  s_p: NH arrays of `stride` >= nkeys floats,
-  // s_red: NH per wave, s_acc: NH * kAttnThreads * 8.  The barriers are the same whatever nkeys is.
-  __device__ __forceinline__ void finish(int nkeys, float scaling, uint16_t *orow, float *s_p, int stride,
-                                         float *s_red, float *s_acc) {
+  // The NH output rows over the nkeys keys at kbase / vbase, value d of row n to store(n, d, o):
+  // o = sum_j p_j v_j[d], or with PART sum_j e^(s_j - mx) v_j[d], unnormalised, and the rows'
+  // maxima and sums (keys that all score -inf weigh nothing: any finite reference).  s_p: NH
+  // arrays of `stride` >= nkeys floats, s_red: NH per wave, s_acc: NH * kAttnThreads * 8.  The
+  // barriers are the same whatever nkeys is.
+  template <bool PART, typename Store>
+  __device__ __forceinline__ void run(int nkeys, float scaling, float *s_p, int stride, float *s_red, float *s_acc,
+                                      Store store, float (&mx)[NH], float (&sum)[NH]) {
     constexpr int kWaves = kAttnThreads / kWave;
     const int npass = kAttnRowsInFlight * rpp;
-    float mx[NH], sum[NH];
 #pragma unroll
     for (int n = 0; n < NH; ++n) {
       mx[n] = -INFINITY;
@@ -135,9 +139,10 @@ struct AttnRow {
     __syncthreads();
 #pragma unroll
     for (int n = 0; n < NH; ++n) {
+      const float mref = PART && mx[n] == -INFINITY ? 0.0f : mx[n];
       sum[n] = 0.0f;
       for (int j = tid; j < nkeys; j += kAttnThreads) {
-        const float e = expf(s_p[n * stride + j] - mx[n]);
+        const float e = expf(s_p[n * stride + j] - mref);
         s_p[n * stride + j] = e;
         sum[n] += e;
       }
@@ -152,10 +157,12 @@ struct AttnRow {
       for (int w = 0; w < kWaves; ++w) sum[n] += s_red[n * kWaves + w];
     }
     __syncthreads();
+    if constexpr (!PART) {
 #pragma unroll
-    for (int n = 0; n < NH; ++n)
-      for (int j = tid; j < nkeys; j += kAttnThreads) s_p[n * stride + j] = bf16r(s_p[n * stride + j] / sum[n]);
-    __syncthreads();
+      for (int n = 0; n < NH; ++n)
+        for (int j = tid; j < nkeys; j += kAttnThreads) s_p[n * stride + j] = bf16r(s_p[n * stride + j] / sum[n]);
+      __syncthreads();
+    }
     // out[d] = sum_j p_j v_j[d]: thread (rr, sub) accumulates dims sub*8 .. sub*8+7 over rows
     // rr, rr + rpp, ... in order; then the rpp partial rows are summed through LDS.
     float acc[NH][8];
@@ -177,12 +184,20 @@ struct AttnRow {
       sa[1] = make_float4(acc[n][4], acc[n][5], acc[n][6], acc[n][7]);
     }
     __syncthreads();
-    for (int i = tid; i < NH * hd; i += kAttnThreads) {
-      const int n = i / hd, d = i - n * hd;
-      float o = 0.0f;
-      for (int r = 0; r < rpp; ++r) o += s_acc[n * kAttnThreads * 8 + r * hd + d];
-      orow[i] = f32_to_bf16(o);
-    }
+#pragma unroll
+    for (int n = 0; n < NH; ++n)
+      for (int d = tid; d < hd; d += kAttnThreads) {
+        float o = 0.0f;
+        for (int r = 0; r < rpp; ++r) o += s_acc[n * kAttnThreads * 8 + r * hd + d];
+        store(n, d, o);
+      }
+  }
+  // The whole of it: NH bf16 rows at `orow`.
+  __device__ __forceinline__ void finish(int nkeys, float scaling, uint16_t *orow, float *s_p, int stride,
+                                         float *s_red, float *s_acc) {
+    float mx[NH], sum[NH];
+    run<false>(nkeys, scaling, s_p, stride, s_red, s_acc,
+               [&](int n, int d, float o) { orow[n * hd + d] = f32_to_bf16(o); }, mx, sum);
   }
 };
 
@@ -199,7 +214,8 @@ attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc
                  MOE_LIST("s"(q), "s"(kc), "s"(vc), "s"(pos0), "s"(out)));
   const int h = blockIdx.x, t = blockIdx.y;
   AttnRow<1> row;
-  row.first(q, kc, vc, nq, nkv, hd, max_seq, h, t, (int)threadIdx.x);
+  row.place(kc, vc, h / (nq / nkv), hd, max_seq, (int)threadIdx.x);
+  row.first(q, nq, h, t, (int)max_seq - 1);
   // Keys 0 .. pos0 + t, bounded by the cache (a position past it is a caller error).
   row.finish(min(*pos0 + t + 1, (int)max_seq), scaling, out + ((size_t)t * nq + h) * hd, s_p, 0, s_red,
              s_acc);
@@ -244,9 +260,11 @@ __device__ __forceinline__ bool attn_last_of(uint32_t *count, int n) {
 // leave at once.
 //
 // Bound: latency (the keys of 3000 tokens are 12 MB, 2 us of HBM).  attention_kernel keeps 32
-// of 256 CUs busy and walks 24 dependent passes there.  One token behind 400 / 1000 / 3000 /
-// 8000 keys: 9.7 / 17.1 / 54.5 / 135 us before, 7.1 / 8.1 / 11.6 / 17.3 us here; 5 tokens
-// behind 2500: 45 and 23 us.  At 250 keys the two are level (6.3 us alone, 7 us shared).
+// of 256 CUs busy and walks 24 dependent passes there.  One token behind 400 / 1000 / 3000
+// keys: 9.7 / 17.1 / 54.4 us so, 7.2 / 8.2 / 11.8 us here; 8 tokens behind 1000 / 3000: 17.6 /
+// 53.1 and 15.7 / 33.6.  Behind a short context the workgroups that leave at once cost 0.25 us
+// (1 / 2 / 8 tokens, nothing cached: 3.9 / 4.0 / 4.1 and 4.2 / 4.2 / 4.4 us; with the token as
+// the slow grid index, behind all splits of the tokens before it, 4.3 / 5.0 / 5.1).
 constexpr int kFewTokens = 8;
 constexpr int kFewSplits = 16;
 constexpr int kFewWhole = 384;
@@ -254,121 +272,50 @@ constexpr int kFewKeys = kAttnMaxKeys / 2;  // of one split, at two splits or mo
 
 __global__ void __launch_bounds__(kAttnThreads)
 few_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restrict__ kc,
-                        const uint16_t *__restrict__ vc, int nq, int nkv, int hd,
+                        const uint16_t *__restrict__ vc, int nq, int nkv, int grp, uint32_t over_nkv, int hd,
                         const int32_t *__restrict__ pos0, int64_t max_seq, float scaling,
                         uint16_t *__restrict__ out, uint32_t *__restrict__ count,
                         float *__restrict__ part) {
   __shared__ float s_p[kFewKeys];
   __shared__ float s_red[kAttnThreads / kWave];
   __shared__ __attribute__((aligned(16))) float s_acc[kAttnThreads * 8];
-  MOE_ARGS_FIRST(MOE_LIST("+s"(nq), "+s"(nkv), "+s"(hd), "+s"(max_seq), "+s"(scaling)),
+  MOE_ARGS_FIRST(MOE_LIST("+s"(nq), "+s"(nkv), "+s"(grp), "+s"(over_nkv), "+s"(hd), "+s"(max_seq), "+s"(scaling)),
                  MOE_LIST("s"(q), "s"(kc), "s"(vc), "s"(pos0), "s"(out), "s"(count), "s"(part)));
   // The KV head is the fast index: a group's query heads read the same cache rows, and with
-  // 8 KV heads they run on one XCD.
-  const int kvh = (int)blockIdx.x % nkv;
-  const int h = kvh * (nq / nkv) + (int)blockIdx.x / nkv;
-  const int split = (int)blockIdx.y, t = (int)blockIdx.z;
-  const int lpr = hd >> 3;
-  const int rpp = kAttnThreads / lpr;
-  const int npass = kAttnRowsInFlight * rpp;
-  const int sub = threadIdx.x & (lpr - 1), rr = threadIdx.x / lpr;
-  float qf[8];
-  unpack8(*reinterpret_cast<const uint4 *>(q + ((size_t)t * nq + h) * hd + sub * 8), qf);
-  const uint16_t *kbase = kc + (size_t)kvh * max_seq * hd + sub * 8;
-  const uint16_t *vbase = vc + (size_t)kvh * max_seq * hd + sub * 8;
-  uint4 kv[kAttnRowsInFlight], vv[kAttnRowsInFlight];
-  auto load_k = [&](int j0, int last) {
-#pragma unroll
-    for (int u = 0; u < kAttnRowsInFlight; ++u)
-      kv[u] = *reinterpret_cast<const uint4 *>(kbase + (size_t)min(j0 + u * rpp + rr, last) * hd);
-  };
-  auto load_v = [&](int j0, int last) {
-#pragma unroll
-    for (int u = 0; u < kAttnRowsInFlight; ++u)
-      vv[u] = *reinterpret_cast<const uint4 *>(vbase + (size_t)min(j0 + u * rpp + rr, last) * hd);
-  };
-  if (split == 0) {  // with q and the position, as in attention_kernel
-    load_k(0, (int)max_seq - 1);
-    load_v(0, (int)max_seq - 1);
-  }
-  const int nkeys = min(*pos0 + t + 1, (int)max_seq);
-  const bool whole = nkeys <= kFewWhole;
-  const int passes = (nkeys + npass - 1) / npass;
-  const int per = (passes + (int)gridDim.y - 1) / (int)gridDim.y;
-  const int nact = whole ? 1 : (passes + per - 1) / per;
-  if (split >= nact) return;  // uniform over the workgroup
-  const int begin = whole ? 0 : split * per * npass;
-  const int end = whole ? nkeys : min(nkeys, begin + per * npass);
-  if (split > 0) {
-    load_k(begin, end - 1);
-    load_v(begin, end - 1);
-  }
-  // Keys count from the split's first below, as the scores in s_p do.
-  const int n = end - begin;
-  float mx = -INFINITY;
-  attn_scores(kv, qf, 0, n, rpp, rr, lpr, sub, scaling, s_p, mx);
-  for (int j0 = npass; j0 < n; j0 += npass) {
-    load_k(begin + j0, end - 1);
-    attn_scores(kv, qf, j0, n, rpp, rr, lpr, sub, scaling, s_p, mx);
-  }
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
-  {
-    float m[1] = {mx};
-    lane_groups_reduce<true>(m, kWave);
-    if (lane == 0) s_red[wave] = m[0];
-    __syncthreads();
-    mx = s_red[0];
-    for (int w = 1; w < kAttnThreads / kWave; ++w) mx = fmaxf(mx, s_red[w]);
-    __syncthreads();
-  }
-  // A split whose scores are all -inf: any finite reference (its probabilities are zero).
-  const float mref = !whole && mx == -INFINITY ? 0.0f : mx;
-  float sum = 0.0f;
-  for (int j = threadIdx.x; j < n; j += kAttnThreads) {
-    const float e = expf(s_p[j] - mref);
-    s_p[j] = e;
-    sum += e;
-  }
-  {
-    float v[1] = {sum};
-    lane_groups_reduce<false>(v, kWave);
-    if (lane == 0) s_red[wave] = v[0];
-    __syncthreads();
-    sum = 0.0f;
-    for (int w = 0; w < kAttnThreads / kWave; ++w) sum += s_red[w];
-    __syncthreads();
-  }
-  if (whole) {
-    for (int j = threadIdx.x; j < n; j += kAttnThreads) s_p[j] = bf16r(s_p[j] / sum);
-    __syncthreads();
-  }
-  float acc[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) acc[e] = 0.0f;
-  attn_pv(vv, 0, n, rpp, rr, s_p, acc);
-  for (int j0 = npass; j0 < n; j0 += npass) {
-    load_v(begin + j0, end - 1);
-    attn_pv(vv, j0, n, rpp, rr, s_p, acc);
-  }
-  float4 *sa = reinterpret_cast<float4 *>(s_acc + rr * hd + sub * 8);
-  sa[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
-  sa[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
-  __syncthreads();
-  // Partials of (token, head): [split][output of hd, maximum, sum].
+  // 8 KV heads they run on one XCD.  The split is the slow one: the first splits, which have
+  // work at any length, start first.
+  const int g = (int)__umulhi(blockIdx.x << 1, over_nkv), kvh = (int)blockIdx.x - g * nkv;
+  const int h = kvh * grp + g;
+  const int t = (int)blockIdx.y, split = (int)blockIdx.z;
   const int unit = t * nq + h;
-  float *const ph = part + (size_t)unit * gridDim.y * (hd + 2);
-  for (int d = threadIdx.x; d < hd; d += kAttnThreads) {
-    float o = 0.0f;
-    for (int r = 0; r < rpp; ++r) o += s_acc[r * hd + d];
-    if (whole)
-      out[(size_t)unit * hd + d] = f32_to_bf16(o);
-    else
-      attn_put(ph + (size_t)split * (hd + 2) + d, o);
+  AttnRow<1> row;
+  row.place(kc, vc, kvh, hd, max_seq, (int)threadIdx.x);
+  if (split == 0) row.first(q, nq, h, t, (int)max_seq - 1);  // with the position, as in attention_kernel
+  const int nkeys = min(*pos0 + t + 1, (int)max_seq);
+  if (nkeys <= kFewWhole) {  // uniform over the workgroup, as what follows
+    if (split == 0) row.finish(nkeys, scaling, out + (size_t)unit * hd, s_p, 0, s_red, s_acc);
+    return;
   }
-  if (whole) return;
+  const int npass = kAttnRowsInFlight * row.rpp;
+  const int passes = (nkeys + npass - 1) / npass;
+  const int per = (passes + (int)gridDim.z - 1) / (int)gridDim.z;
+  const int nact = (passes + per - 1) / per;
+  if (split >= nact) return;
+  const int begin = split * per * npass;
+  const int n = min(nkeys - begin, per * npass);
+  if (split > 0) {
+    row.kbase += (size_t)begin * hd;
+    row.vbase += (size_t)begin * hd;
+    row.first(q, nq, h, t, n - 1);
+  }
+  // Partials of (token, head): [split][output of hd, maximum, sum].
+  float *const ph = part + (size_t)unit * gridDim.z * (hd + 2);
+  float *const mine = ph + (size_t)split * (hd + 2);
+  float mx[1], sum[1];
+  row.run<true>(n, scaling, s_p, 0, s_red, s_acc, [&](int, int d, float o) { attn_put(mine + d, o); }, mx, sum);
   if (threadIdx.x == 0) {
-    attn_put(ph + (size_t)split * (hd + 2) + hd, mx);
-    attn_put(ph + (size_t)split * (hd + 2) + hd + 1, sum);
+    attn_put(mine + hd, mx[0]);
+    attn_put(mine + hd + 1, sum[0]);
   }
   if (!attn_last_of(count + unit, nact)) return;
   // Weights of the splits (and the sum's share of each) in LDS, then the outputs, all loads
@@ -544,7 +491,8 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
     const int unit = min(2 * wg + half, units - 1);  // (an odd last unit twice, the same values)
     const int t = unit / (nq / ROWS), h = (unit - t * (nq / ROWS)) * ROWS;
     AttnRow<ROWS> row;
-    row.first(q, kc, vc, nq, nkv, HD, max_seq, h, t, (int)threadIdx.x & (kAttnThreads - 1));
+    row.place(kc, vc, h / (nq / nkv), HD, max_seq, (int)threadIdx.x & (kAttnThreads - 1));
+    row.first(q, nq, h, t, (int)max_seq - 1);
     const int p0 = *pos0;
     if (min(p0 + T, (int)max_seq) <= kFaRowKeys) {
       if (2 * wg >= units) return;
@@ -919,7 +867,8 @@ AttnPlan attn_plan(int64_t T, int32_t nq, int32_t nkv, int32_t hd, int64_t max_s
       if (p.splits > 1) p.bytes = kAttnCounterBytes + p.units * p.splits * 4 * (hd / 2 + 2) * kWave * 4;
     }
   } else if (T <= kFewTokens && ws && max_seq > kFewWhole && (hd == 64 || hd == 128 || hd == 256)) {
-    // Two workgroups per CU: those that leave at once behind a short context cost 0.1 us (four: 0.4).
+    // Two workgroups per CU: those that leave at once behind a short context cost 0.25 us (half as
+    // many splits 0.2, and 12.3 instead of 11.8 us behind 3000 keys).
     const int64_t pass = kAttnRowsInFlight * (kAttnThreads / (hd / 8));
     const int64_t most = (max_seq + pass - 1) / pass;
     int64_t s = 2 * (int64_t)device_cu_count() / (nq * T);
@@ -1004,9 +953,12 @@ extern "C" int moe_attention_ws_bf16(const void *q, const void *k_cache, const v
     hipLaunchKernelGGL(kern, dim3((unsigned)p.units, y), dim3(moe::kFaThreads), 0, s, qp, kp, vp, (int)T,
                        n_q_heads, n_kv_heads, pp, max_seq, scaling, op, count, part, p.splits);
   } else if (!p.matrix && p.splits > 1) {
-    hipLaunchKernelGGL(moe::few_attention_kernel, dim3((unsigned)n_q_heads, (unsigned)p.splits, (unsigned)T),
-                       dim3(moe::kAttnThreads), 0, s, qp, kp, vp, n_q_heads, n_kv_heads, head_dim, pp,
-                       max_seq, scaling, op, count, part);
+    // grp = nq / nkv and x / nkv = (x * over_nkv) >> 31 (exact: x < nq <= kAttnUnitsMax), so that
+    // no division stands before the kernel's first loads.
+    const uint32_t over_nkv = (uint32_t)((((int64_t)1 << 31) + n_kv_heads - 1) / n_kv_heads);
+    hipLaunchKernelGGL(moe::few_attention_kernel, dim3((unsigned)n_q_heads, (unsigned)T, (unsigned)p.splits),
+                       dim3(moe::kAttnThreads), 0, s, qp, kp, vp, n_q_heads, n_kv_heads,
+                       n_q_heads / n_kv_heads, over_nkv, head_dim, pp, max_seq, scaling, op, count, part);
   } else {
     hipLaunchKernelGGL(moe::attention_kernel, dim3((unsigned)n_q_heads, (unsigned)T),
                        dim3(moe::kAttnThreads), 0, s, qp, kp, vp, n_q_heads, n_kv_heads, head_dim, pp,

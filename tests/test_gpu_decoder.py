@@ -162,7 +162,8 @@ def _attend_ref(q, k, v, p0, scaling=None):
     (129, 0, 256, 16, 2, 64), (65, 127, 200, 24, 4, 128), (66, 64, 130, 16, 16, 128),
     (100, 0, 128, 16, 4, 128), (60, 0, 64, 32, 8, 64), (60, 68, 128, 32, 8, 128),
     (16, 368, 400, 32, 8, 128), (16, 369, 400, 32, 8, 128), (9, 5, 64, 7, 7, 64),
-    (30, 300, 400, 32, 4, 128), (17, 3, 64, 34, 17, 64)])
+    (30, 300, 400, 32, 4, 128), (17, 3, 64, 34, 17, 64),
+    (3, 700, 1024, 6, 1, 128), (8, 300, 1024, 21, 7, 64), (2, 900, 1024, 5, 5, 256)])
 def test_attention_forms(cuda_device, T, p0, max_seq, nq, nkv, hd):
     """Matrix form and shared keys: against the module's arithmetic, with cache rows past the
     last key NaN; the workspace's counters return to zero, a second call repeats the bits."""
