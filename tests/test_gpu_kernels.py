@@ -71,8 +71,9 @@ def test_quantize_bitexact(cuda_device, shape):
 @pytest.mark.parametrize("case", ["nf4", "crowded", "unsorted", "nan_code"])
 @pytest.mark.parametrize("chunks", [1, 2, 8192 + 3])
 def test_quantize_binned_is_general(cuda_device, case, chunks):
-    """The blocksize-64 kernel (midpoints counted through a table of bins) against the general
-    one (every midpoint compared), for any codebook and any weights: bit for bit."""
+    """The blocksize-64 kernel (one or two chunks: every midpoint compared; more than a chunk a
+    wave: midpoints counted through a table of bins) against the general one, for any codebook
+    and any weights: bit for bit."""
     from moeinfra_amd import _lib, ops
 
     code = torch.from_numpy(orc.NF4_CODE.copy())
