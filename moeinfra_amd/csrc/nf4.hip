@@ -74,9 +74,8 @@ constexpr int kQuantThreads = 256;
 // now comes from a table of 64 equal bins over [-1, 1].  A bin index is monotone in y, so
 // midpoints in lower bins are below y and those in higher bins are not; a bin holds at most
 // one midpoint of a codebook like NF4's (their distance is at least 2.5 bins), against which
-// one comparison decides: 36 us
-// (4.1 TB/s; 48 us while every thread built eight table entries and no load ran ahead).  The
-// entry {midpoint, count below the bin} has 32 replicas
+// one comparison decides: 32 to 34 us (4.5 TB/s; 48 us while every thread built eight table
+// entries and no load ran ahead).  The entry {midpoint, count below the bin} has 32 replicas
 // (conflict-free ds_read_b64).  A codebook with two midpoints in a bin compares with all 15.
 // So do weights with at most one chunk a wave (TABLE false): every workgroup builds the table for
 // itself, half a microsecond that one chunk does not earn back (512 / 1 M / 4 M values: 3.2 / 4.0
