@@ -493,7 +493,7 @@ prefill_attention_kernel(const uint16_t *__restrict__ q, const uint16_t *__restr
     AttnRow<ROWS> row;
     row.place(kc, vc, h / (nq / nkv), HD, max_seq, (int)threadIdx.x & (kAttnThreads - 1));
     row.first(q, nq, h, t, (int)max_seq - 1);
-    const int p0 = *pos0;
+    const int p0 = min(*pos0, (int)max_seq);  // (a position past the cache is a caller error)
     if (min(p0 + T, (int)max_seq) <= kFaRowKeys) {
       if (2 * wg >= units) return;
       float *const s_acc = reinterpret_cast<float *>(&s_kv[0][0][0]) + half * kUnit;
